@@ -58,14 +58,9 @@ int ssxk_ns_div(void *st, size_t nt, const double *const J[9],
 int ssxk_ns_grad(void *st, size_t nt, int n, const double *dm,
 		const double *p, const double *mass, const double *const ti[9],
 		double *const out[3]);
-int ssxk_ns_conv(void *st, size_t nt, int n, const double *dm,
-		const double *const u[3], const double *const v[3],
-		const double *const Jv[9], const double *const ti[9],
-		const double *mass, double *const out[3]);
-size_t ssxk_ns_conv_full_bytes(int n, int nc);
-int ssxk_ns_conv_full(void *st, int nel, int n, int nc, const double *prol,
+int ssxk_ns_conv(void *st, int nel, int n, const double *prol,
 		const double *dm, const double *const u[3], const double *const v[3],
-		const double *const ti[9], const double *mass, double *const out[3]);
+		const double *geo, double *const out[3]);
 int ssxk_ns_surf(void *st, int nel, int n, const int *bc, int dirichlet,
 		const double *wn, const double *g, double *f);
 int ssxk_ns_zero_dir(void *st, size_t nt, int n, const int *bc,
@@ -85,15 +80,12 @@ struct ssx_ns {
 	/* geometry: level 0 (tinv, face weights x normals per direction) and
 	 * the convective level */
 	double *ti[9], *wn[3];
-	double *dm_c, *prol_c, *ti_c[9], *mass_c;
+	double *dm_c, *prol_c, *geo_c;   /* geo_c: [e][9][nc^3] w detJ dxi_b/dx_a */
 	/* fields: [0] newest level */
 	double *u[3][3], *p[3], *conv[3][3], *rot[3][3];
 	/* scratch at n */
 	double *ut[3], *rhs[3], *a[3], *b[3], *J[9];
 	double *rkf[4][3], *rky[4][3];
-	/* scratch at nconv */
-	double *cu[3], *cv[3], *cJ[9], *co[3];
-	int conv_elem;               /* convection one workgroup per element */
 	int inited;
 	long long cnt_solve[4];
 };
@@ -121,10 +113,8 @@ void ssx_ns_destroy(ssx_ns *ns)
 		return;
 	if (ns->vb)
 		ssx_batch_destroy(ns->vb);
-	double **all[] = { ns->ti, ns->ti + 3, ns->ti + 6, ns->wn, ns->ti_c,
-		ns->ti_c + 3, ns->ti_c + 6, ns->ut, ns->rhs, ns->a, ns->b, ns->J,
-		ns->J + 3, ns->J + 6, ns->cu, ns->cv, ns->cJ, ns->cJ + 3, ns->cJ + 6,
-		ns->co, ns->p };
+	double **all[] = { ns->ti, ns->ti + 3, ns->ti + 6, ns->wn, ns->ut,
+		ns->rhs, ns->a, ns->b, ns->J, ns->J + 3, ns->J + 6, ns->p };
 	for (size_t k = 0; k < sizeof(all) / sizeof(all[0]); ++k)
 		for (int c = 0; c < 3; ++c)
 			hipFree(all[k][c]);
@@ -141,7 +131,7 @@ void ssx_ns_destroy(ssx_ns *ns)
 		}
 	hipFree(ns->dm_c);
 	hipFree(ns->prol_c);
-	hipFree(ns->mass_c);
+	hipFree(ns->geo_c);
 	free(ns);
 }
 
@@ -268,18 +258,30 @@ static int ns_geometry(ssx_ns *ns)
 				}
 		}
 	ssx_jacobians(&bc, nel, xc[0], xc[1], xc[2], jac, jinv, det);
-	for (int a = 0; a < 3 && rc == SSX_OK; ++a)
-		for (int b = 0; b < 3 && rc == SSX_OK; ++b)
-			rc = nup(&ns->ti_c[3 * a + b], jinv[3 * b + a], ntc);
-	for (int e = 0; e < nel; ++e)
-		for (int k = 0; k < nc; ++k)
-			for (int j = 0; j < nc; ++j)
-				for (int i = 0; i < nc; ++i) {
-					const size_t q = (size_t) e * nc3 + (k * nc + j) * nc + i;
-					det[q] = (bc.rho[i] * bc.rho[j] * bc.rho[k]) * det[q];
-				}
-	if (rc == SSX_OK)
-		rc = nup(&ns->mass_c, det, ntc);
+	/* w detJ d xi_b / d x_a, element by element */
+	{
+		double *geo = malloc(sizeof(double) * 9 * ntc);
+		if (!geo) {
+			ssx_set_error("out of host memory (Navier-Stokes geometry)");
+			rc = SSX_ENOMEM;
+		}
+		for (int e = 0; e < nel && geo; ++e)
+			for (int k = 0; k < nc; ++k)
+				for (int j = 0; j < nc; ++j)
+					for (int i = 0; i < nc; ++i) {
+						const int r = (k * nc + j) * nc + i;
+						const size_t q = (size_t) e * nc3 + r;
+						const double wj = (bc.rho[i] * bc.rho[j] * bc.rho[k])
+							* det[q];
+						for (int a = 0; a < 3; ++a)
+							for (int b = 0; b < 3; ++b)
+								geo[((size_t) e * 9 + 3 * a + b) * nc3 + r] =
+									wj * jinv[3 * b + a][q];
+					}
+		if (rc == SSX_OK)
+			rc = nup(&ns->geo_c, geo, 9 * ntc);
+		free(geo);
+	}
 	if (rc == SSX_OK)
 		rc = nup(&ns->dm_c, bc.d, (size_t) nc * nc);
 	if (rc == SSX_OK)
@@ -337,19 +339,8 @@ int ssx_ns_create(ssx_ns **out, ssx_ctx *c, const ssx_ns_params *prm)
 	for (int d = 0; d < 3; ++d)
 		ns->g[d] = prm->g[d];
 	ns->batched = prm->batch_velocity;
-	/* the whole convection operator one element per workgroup where its
-	 * LDS fits the device, else the transfer kernels and the node-per-lane
-	 * operator with the Jacobian of v stored (cJ) */
-	{
-		int dev = 0, lim = 0;
-		const size_t need = ssxk_ns_conv_full_bytes(n, nc);
-		ns->conv_elem = hipGetDevice(&dev) == hipSuccess
-			&& hipDeviceGetAttribute(&lim,
-					hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess
-			&& need <= (size_t) lim;
-	}
 	int rc = ns_geometry(ns);
-	const size_t nt = ns->nt, ntc = ns->ntc;
+	const size_t nt = ns->nt;
 	for (int l = 0; l < 3 && rc == SSX_OK; ++l)
 		for (int d = 0; d < 3 && rc == SSX_OK; ++d) {
 			rc = nalloc(&ns->u[l][d], nt);
@@ -360,22 +351,17 @@ int ssx_ns_create(ssx_ns **out, ssx_ctx *c, const ssx_ns_params *prm)
 		}
 	for (int d = 0; d < 3 && rc == SSX_OK; ++d) {
 		double **v[] = { &ns->p[d], &ns->ut[d], &ns->rhs[d], &ns->a[d],
-			&ns->b[d], &ns->cu[d], &ns->cv[d], &ns->co[d] };
-		const size_t sz[] = { nt, nt, nt, nt, nt, ntc, ntc, ntc };
-		/* the nc-point fields only for the unfused convection */
-		for (int k = 0; k < (ns->conv_elem ? 5 : 8) && rc == SSX_OK; ++k)
-			rc = nalloc(v[k], sz[k]);
+			&ns->b[d] };
+		for (int k = 0; k < 5 && rc == SSX_OK; ++k)
+			rc = nalloc(v[k], nt);
 		for (int s = 0; s < 4 && rc == SSX_OK; ++s) {
 			rc = nalloc(&ns->rkf[s][d], nt);
 			if (rc == SSX_OK)
 				rc = nalloc(&ns->rky[s][d], nt);
 		}
 	}
-	for (int k = 0; k < 9 && rc == SSX_OK; ++k) {
+	for (int k = 0; k < 9 && rc == SSX_OK; ++k)
 		rc = nalloc(&ns->J[k], nt);
-		if (rc == SSX_OK && !ns->conv_elem)
-			rc = nalloc(&ns->cJ[k], ntc);
-	}
 	/* zero histories (the element constructor's zeroed arrays) */
 	for (int l = 0; l < 3 && rc == SSX_OK; ++l) {
 		rc = ssxk_fill(c->stream, ns->p[l], 0.0, nt);
@@ -419,25 +405,9 @@ static void rotate3(double *h[3][3])
 static int ns_convection(ssx_ns *ns, double *const u[3], double *const v[3],
 		double *const out[3])
 {
-	void *st = ns->c->stream;
-	const int n = ns->n, nc = ns->nc, nel = ns->nel;
-	if (ns->conv_elem)          /* the whole operator per element */
-		return ssxk_ns_conv_full(st, nel, n, nc, ns->prol_c, ns->dm_c,
-				(const double *const *) u, (const double *const *) v,
-				(const double *const *) ns->ti_c, ns->mass_c, out);
-	for (int d = 0; d < 3; ++d) {
-		TRYN(ssxk_prolong(st, nc, n, nel, ns->prol_c, u[d], ns->cu[d], 0));
-		TRYN(ssxk_prolong(st, nc, n, nel, ns->prol_c, v[d], ns->cv[d], 0));
-	}
-	TRYN(ssxk_ns_jac(st, ns->ntc, nc, ns->dm_c, (const double *const *) ns->cv,
-			ns->cJ));
-	TRYN(ssxk_ns_conv(st, ns->ntc, nc, ns->dm_c,
-			(const double *const *) ns->cu, (const double *const *) ns->cv,
-			(const double *const *) ns->cJ, (const double *const *) ns->ti_c,
-			ns->mass_c, ns->co));
-	for (int d = 0; d < 3; ++d)
-		TRYN(ssxk_restrict(st, nc, n, nel, ns->prol_c, ns->co[d], out[d]));
-	return SSX_OK;
+	return ssxk_ns_conv(ns->c->stream, ns->nel, ns->n, ns->prol_c, ns->dm_c,
+			(const double *const *) u, (const double *const *) v, ns->geo_c,
+			out);
 }
 
 /* double_curl_operator (stokes.c:94-105) -> out */

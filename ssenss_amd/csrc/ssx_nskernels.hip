@@ -157,334 +157,367 @@ k_ns_grad(long long nt, int n, const double *__restrict__ dm,
 	}
 }
 
-// skew-symmetric convection at the convective resolution
-// (skew_symmetric_convection_operator, convection.c:129-140): half the
-// convective form (u . grad) v_c (convective_convection_operator, :71-93)
-// plus half the conservative form as convection.c:95-127 forms it,
-// sum_a sum_b (d xi_b/d x_a) D_b(u_b v_c), each times w detJ
-__global__ void __launch_bounds__(256)
-k_ns_conv(long long nt, int n, const double *__restrict__ dm, P3 u, P3 v,
-		P9 Jv, P9 ti, const double *__restrict__ mass, M3 out)
+// ---------------------------------------------------------------------
+// The dealiased skew-symmetric convection operator, one workgroup per
+// element (antialiased_convection_operator, convection.c:37-69): u and v
+// interpolated from N to NC = 3N/2 points, half the convective form
+// (u . grad) v_c (:71-93) plus half the conservative form as
+// convection.c:95-127 forms it, sum_a sum_b (d xi_b/d x_a) D_b(u_b v_c),
+// each times w detJ, integrated back to N points.
+//
+// Every contraction (interpolation, D, and their transposes) is a product
+// of a small constant matrix with the element's lines, taken by the FP64
+// matrix instruction 16x16x4: the constant matrix sits in registers (one
+// value a lane and step of 4), the lines come from LDS once each, so LDS
+// carries one read and one write per value and contraction.  The earlier
+// form (one lane a node, matrix and lines read from LDS at every
+// multiply-add) was LDS-bound.
+//
+// With C_b = sum_a u_a g_ab and T_b = sum_a g_ab, g_ab = w detJ d xi_b/d x_a
+// (premultiplied at set-up), both forms together are
+//   0.5 sum_b (C_b D_b v_c + T_b D_b(u_b v_c)),
+// so the nine factors are read once, in the lane layout in which the
+// matrix instruction leaves D_b's result (another for each direction b:
+// 36 loads a lane), and the three components take them from registers;
+// the directions meet in LDS.  One wavefront a tile of 16 lines, W =
+// ceil(NC^2 / 16) of them (960 lanes at NC = 15); LDS 6 NC^2 (NC|1)
+// doubles: one workgroup a CU at N = 10.
+//
+// What bounds it at N = 10: 12 short phases between barriers of the one
+// workgroup a CU holds.  The matrix instructions (2050 of them an element,
+// 0.5 ms on 9216 elements at their peak) keep their unit busy 38 % of the
+// time and the address arithmetic its own 26 %; the factors (2.2 GB) are
+// loaded during the contractions of u.  Measured per evaluation: 9216
+// elements at N = 10 3.5 -> 1.47 ms, 64 elements at N = 8 48 -> 24 us.
+// ---------------------------------------------------------------------
+typedef double conv_v4 __attribute__((ext_vector_type(4)));
+
+template <int N, int NC>
+struct ConvShape {
+	static constexpr int W = (NC * NC + 15) / 16;   // wavefronts
+	static constexpr int KP = N | 1, KC = NC | 1;   // odd LDS rows
+	static constexpr int REG = 3 * NC * NC * KC;    // doubles of a region
+	static constexpr size_t BYTES = sizeof(double) * (2 * REG + 64);
+};
+
+// D's rows of the 16x16x4 instruction: lane l holds rows 4 r + l / 16 (r =
+// 0..3) of column l % 16; A: row l % 16, k = l / 16; B: column l % 16, k =
+// l / 16
+#define CONV_ROW(r) (4 * (r) + kq)
+
+// the same value, hidden from the compiler: it would otherwise compute the
+// addresses of every phase from the lane number once, keep them in
+// registers throughout and spill (97 registers at N = 10)
+__device__ __forceinline__ int fresh(int x)
 {
-	const long long q = (long long) blockIdx.x * 256 + threadIdx.x;
-	if (q >= nt)
-		return;
-	const int n3 = n * n * n;
-	const long long e = q / n3;
-	const int r = (int) (q - e * n3);
-	const int i = r % n, j = (r / n) % n, k = r / (n * n);
-	const long long b0 = e * n3;
-	double tv[9], uq[3];
-	for (int a = 0; a < 9; ++a)
-		tv[a] = ti.p[a][q];
-	for (int a = 0; a < 3; ++a)
-		uq[a] = u.p[a][q];
-	const double wj = mass[q];
-	for (int c = 0; c < 3; ++c) {
-		// convective: dv_ci = sum_k tinv[i][k] D_k v_c; sum_i u_i dv_ci
-		double cv = 0.0;
-		for (int a = 0; a < 3; ++a) {
-			double dv = 0.0;
-			for (int b = 0; b < 3; ++b) {
-				const double t = tv[3 * a + b] * Jv.p[3 * c + b][q];
-				dv = b == 0 ? t : t + dv;
-			}
-			const double t = uq[a] * dv;
-			cv = a == 0 ? t : t + cv;
-		}
-		cv = cv * wj;
-		// conservative: tmp_b = D_b(u_b v_c); duvd_a = sum_b tinv[a][b]
-		// tmp_b; sum over a
-		double tb[3] = { 0.0, 0.0, 0.0 };
-		for (int l = 0; l < n; ++l) {
-			const long long qx = b0 + (k * n + j) * n + l;
-			const long long qy = b0 + (k * n + l) * n + i;
-			const long long qz = b0 + (l * n + j) * n + i;
-			tb[0] += dm[i * n + l] * (u.p[0][qx] * v.p[c][qx]);
-			tb[1] += dm[j * n + l] * (u.p[1][qy] * v.p[c][qy]);
-			tb[2] += dm[k * n + l] * (u.p[2][qz] * v.p[c][qz]);
-		}
-		double cs = 0.0;
-		for (int a = 0; a < 3; ++a) {
-			double d = 0.0;
-			for (int b = 0; b < 3; ++b) {
-				const double t = tv[3 * a + b] * tb[b];
-				d = b == 0 ? t : t + d;
-			}
-			cs = a == 0 ? d : cs + d;
-		}
-		cs = cs * wj;
-		out.p[c][q] = 0.5 * cs + 0.5 * cv;
-	}
+	asm volatile("" : "+v"(x));
+	return x;
 }
 
-// The same operator, one workgroup per element: the three u components
-// and one v component at a time are staged in LDS, so the reference
-// derivatives of v and of u_b v along every line come from LDS instead of
-// per-node global gathers, and the Jacobian of v is never stored.  Per
-// node and component the arithmetic is k_ns_conv's (dref's sums, then the
-// same combinations).  LDS: 4 n^3 + n^2 doubles (n <= 15).
-__global__ void __launch_bounds__(1024)
-k_ns_conv_elem(int n, const double *__restrict__ dm, P3 u, P3 v, P9 ti,
-		const double *__restrict__ mass, M3 out)
+// one contraction of three components: for every line l < C of component f,
+// dst(f, l)[m * SM] = sum_k a[m][k] src(f, l)[k], m < M, k < K.  A
+// wavefront takes its tiles of 16 lines together (all loads, then the
+// matrix instructions in turn), with no branch: lines and rows past the end
+// read the last line and write to `dump` (DUMP false: not at all).
+template <int M, int K, int C, int SM, int W, bool DUMP, typename Src,
+		typename Dst>
+__device__ __forceinline__ void conv_stage(const double *a, int wave,
+		int lane, double *dump, Src src, Dst dst)
 {
+	constexpr int KS = (K + 3) / 4, TI = ((3 * C + 15) / 16 + W - 1) / W;
+	const int l = fresh(lane), col = l & 15, kq = l >> 4;
+	const int klast = 4 * (KS - 1) + kq < K ? 4 * (KS - 1) + kq : K - 1;
+	double b[TI][KS];
+	double *o[TI];
+	bool ok[TI];
+	conv_v4 d[TI];
+#pragma unroll
+	for (int t = 0; t < TI; ++t) {
+		const int q0 = 16 * (wave + t * W) + col;
+		const int q = q0 < 3 * C ? q0 : 3 * C - 1;
+		const int f = q / C, c = q - f * C;
+		const double *p = src(f, c);
+#pragma unroll
+		for (int s = 0; s < KS; ++s)
+			b[t][s] = p[s < KS - 1 ? 4 * s + kq : klast];
+		ok[t] = q0 < 3 * C;
+		o[t] = dst(f, c) + kq * SM;
+	}
+	// every load issued before the first is used, none behind a branch
+#pragma unroll
+	for (int t = 0; t < TI; ++t) {
+#pragma unroll
+		for (int s = 0; s < KS; ++s)
+			asm volatile("" : "+v"(b[t][s]));
+		if (K % 4 != 0)
+			b[t][KS - 1] = 4 * (KS - 1) + kq < K ? b[t][KS - 1] : 0.0;
+		d[t] = conv_v4{ 0.0, 0.0, 0.0, 0.0 };
+	}
+#pragma unroll
+	for (int s = 0; s < KS; ++s)
+#pragma unroll
+		for (int t = 0; t < TI; ++t)
+			d[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], b[t][s], d[t],
+					0, 0, 0);
+#pragma unroll
+	for (int t = 0; t < TI; ++t)
+#pragma unroll
+		for (int r = 0; r < 4; ++r) {
+			if (4 * r >= M)
+				continue;
+			const bool in = ok[t] && (4 * r + 3 < M || CONV_ROW(r) < M);
+			if (DUMP)
+				*(in ? o[t] + 4 * r * SM : dump) = d[t][r];
+			else if (in)
+				o[t][4 * r * SM] = d[t][r];
+		}
+}
+
+template <int N, int NC>
+__global__ void __launch_bounds__((64 * ConvShape<N, NC>::W))
+k_ns_conv(const double *__restrict__ prol, const double *__restrict__ dm,
+		P3 u, P3 v, const double *__restrict__ geo, M3 out)
+{
+	using S = ConvShape<N, NC>;
+	constexpr int W = S::W, KP = S::KP, KC = S::KC;
+	constexpr int N2 = N * N, N3 = N2 * N, C2 = NC * NC, C3 = C2 * NC;
+	constexpr int F3 = C2 * KC;             // one field at NC points in LDS
+	constexpr int SP = (N + 3) / 4, SC = (NC + 3) / 4;
 	extern __shared__ double sm[];
-	const int n2 = n * n, n3 = n2 * n;
-	double *su = sm;                    // u_0, u_1, u_2
-	double *sv = sm + 3 * n3;           // v_c
-	double *sd = sm + 4 * n3;           // D
-	const long long b0 = (long long) blockIdx.x * n3;
-	for (int q = threadIdx.x; q < n2; q += blockDim.x)
-		sd[q] = dm[q];
-	for (int a = 0; a < 3; ++a)
-		for (int q = threadIdx.x; q < n3; q += blockDim.x)
-			su[a * n3 + q] = u.p[a][b0 + q];
-	for (int c = 0; c < 3; ++c) {
-		__syncthreads();                // sv free (c > 0), su/sd ready
-		for (int q = threadIdx.x; q < n3; q += blockDim.x)
-			sv[q] = v.p[c][b0 + q];
-		__syncthreads();
-		for (int r = threadIdx.x; r < n3; r += blockDim.x) {
-			const int i = r % n, j = (r / n) % n, k = r / n2;
-			const long long q = b0 + r;
-			// D_b v_c, b = xi, eta, zeta (dref's order)
-			double jv[3] = { 0.0, 0.0, 0.0 };
-			double tb[3] = { 0.0, 0.0, 0.0 };
-			const double *rx = sv + (k * n + j) * n;
-			const double *ry = sv + k * n2 + i;
-			const double *rz = sv + j * n + i;
-			const double *ux = su + (k * n + j) * n;
-			const double *uy = su + n3 + k * n2 + i;
-			const double *uz = su + 2 * n3 + j * n + i;
-			for (int l = 0; l < n; ++l) {
-				jv[0] += sd[i * n + l] * rx[l];
-				jv[1] += sd[j * n + l] * ry[l * n];
-				jv[2] += sd[k * n + l] * rz[l * n2];
-				tb[0] += sd[i * n + l] * (ux[l] * rx[l]);
-				tb[1] += sd[j * n + l] * (uy[l * n] * ry[l * n]);
-				tb[2] += sd[k * n + l] * (uz[l * n2] * rz[l * n2]);
-			}
-			double tv[9];
+	double *ra = sm, *rb = sm + S::REG;
+	double *dump = sm + 2 * S::REG + (threadIdx.x & 63);
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	const int col = lane & 15, kq = lane >> 4;
+	const size_t e = blockIdx.x;
+	// the interpolation matrix (rows < NC, k < N), zero outside; D and the
+	// transpose are loaded where they are used, to keep registers free
+	double ap[SP];
 #pragma unroll
-			for (int a = 0; a < 9; ++a)
-				tv[a] = ti.p[a][q];
-			const double wj = mass[q];
-			double cv = 0.0;
-#pragma unroll
-			for (int a = 0; a < 3; ++a) {
-				double dv = 0.0;
-#pragma unroll
-				for (int b = 0; b < 3; ++b) {
-					const double t = tv[3 * a + b] * jv[b];
-					dv = b == 0 ? t : t + dv;
-				}
-				const double t = su[a * n3 + r] * dv;
-				cv = a == 0 ? t : t + cv;
-			}
-			cv = cv * wj;
-			double cs = 0.0;
-#pragma unroll
-			for (int a = 0; a < 3; ++a) {
-				double d = 0.0;
-#pragma unroll
-				for (int b = 0; b < 3; ++b) {
-					const double t = tv[3 * a + b] * tb[b];
-					d = b == 0 ? t : t + d;
-				}
-				cs = a == 0 ? d : cs + d;
-			}
-			cs = cs * wj;
-			out.p[c][q] = 0.5 * cs + 0.5 * cv;
+	for (int s = 0; s < SP; ++s) {
+		const int k = 4 * s + kq;
+		const bool ok = col < NC && k < N;
+		const double x = prol[ok ? k * NC + col : 0];
+		ap[s] = ok ? x : 0.0;
+	}
+	// this wavefront's lines: line c of tile `wave` along eta (z, x), zeta
+	// (y, x) by column, along xi (z, y) by row; idle lanes take line 0
+	struct Line { int col, kq, c, cz, ci; bool ok; };
+	auto line = [&]() {
+		const int l = fresh(lane);
+		Line w;
+		w.col = l & 15;
+		w.kq = l >> 4;
+		const int cl = 16 * wave + w.col;
+		w.ok = cl < C2;
+		w.c = w.ok ? cl : 0;
+		w.cz = w.c / NC;
+		w.ci = w.c - w.cz * NC;
+		return w;
+	};
+
+	// three contractions: interpolation of w (global) to NC points in ra
+	// ([X][z][y], then [Y][X][z], then [Z][Y][X])
+	auto interpolate = [&](const P3 &w, auto &&loads) {
+		const double *w0 = w.p[0] + e * N3, *w1 = w.p[1] + e * N3,
+			*w2 = w.p[2] + e * N3;
+		conv_stage<NC, N, N2, N * KP, W, true>(ap, wave, lane, dump,
+			[&](int f, int l) {
+				return (f == 0 ? w0 : f == 1 ? w1 : w2) + l * N;
+			},
+			[&](int f, int l) {
+				return ra + f * (NC * N * KP) + (l / N) * KP + l % N;
+			});
+		loads();
+		lds_sync();
+		conv_stage<NC, N, NC * N, NC * KP, W, true>(ap, wave, lane, dump,
+			[&](int f, int l) { return ra + f * (NC * N * KP) + l * KP; },
+			[&](int f, int l) {
+				return rb + f * (C2 * KP) + (l / N) * KP + l % N;
+			});
+		lds_sync();
+		conv_stage<NC, N, C2, NC * KC, W, true>(ap, wave, lane, dump,
+			[&](int f, int l) { return rb + f * (C2 * KP) + l * KP; },
+			[&](int f, int l) {
+				return ra + f * F3 + (l / NC) * KC + l % NC;
+			});
+		lds_sync();
+	};
+
+	// node of this lane's result r along direction b, as line (z, y) and x:
+	// along xi the rows are lines and the columns x (idle lanes: node 0)
+	auto result = [&](const Line &w, int b, int r, int &zy, int &x) {
+		const int m = 4 * r + w.kq;
+		if (b == 0) {
+			const int l = 16 * wave + m;
+			const bool ok = l < C2 && w.col < NC;
+			zy = ok ? l : 0;
+			x = ok ? w.col : 0;
+		} else {
+			const int mm = w.ok && m < NC ? m : 0;
+			zy = b == 1 ? w.cz * NC + mm : mm * NC + w.cz;
+			x = w.ci;
 		}
-	}
-}
+	};
 
-// The whole dealiased operator of one element in one workgroup
-// (antialiased_convection_operator, convection.c:37-69): u and v are
-// interpolated from n to nc points into LDS (interpolate_to_grid, the three
-// contractions of k_prolong), the skew-symmetric operator is formed at the
-// nc points as in k_ns_conv_elem, and each component is integrated back to
-// n points (integrate_to_grid, the contractions of k_restrict).  Every sum
-// runs in the order of those kernels.  prol[p*nc+i] = l_p(xi_i) (p < n
-// coarse, i < nc fine).
-#define CONV_SCR(n, nc) ((n) * (n) * (n) + (n) * (n) * (nc) + (n) * (nc) * (nc))
-
-// dst[nc^3] = the interpolation to nc points of src[n^3] (global); scr:
-// CONV_SCR doubles
-__device__ __forceinline__ void conv_prolong(int n, int nc,
-		const double *__restrict__ sp, const double *__restrict__ src,
-		double *__restrict__ dst, double *__restrict__ scr)
-{
-	double *in = scr, *t1 = scr + n * n * n, *t2 = t1 + n * n * nc;
-	const int n3 = n * n * n;
-	for (int q = threadIdx.x; q < n3; q += blockDim.x)
-		in[q] = src[q];
-	__syncthreads();
-	for (int q = threadIdx.x; q < n * n * nc; q += blockDim.x) {
-		const int i = q % nc, kj = q / nc;
-		double s = 0.0;
-		for (int p = 0; p < n; ++p)
-			s += sp[p * nc + i] * in[kj * n + p];
-		t1[q] = s;
-	}
-	__syncthreads();
-	for (int q = threadIdx.x; q < n * nc * nc; q += blockDim.x) {
-		const int i = q % nc, jq = (q / nc) % nc, k = q / (nc * nc);
-		double s = 0.0;
-		for (int l = 0; l < n; ++l)
-			s += t1[(k * n + l) * nc + i] * sp[l * nc + jq];
-		t2[q] = s;
-	}
-	__syncthreads();
-	for (int q = threadIdx.x; q < nc * nc * nc; q += blockDim.x) {
-		const int ji = q % (nc * nc), k = q / (nc * nc);
-		double s = 0.0;
-		for (int l = 0; l < n; ++l)
-			s += t2[l * nc * nc + ji] * sp[l * nc + k];
-		dst[q] = s;
-	}
-	__syncthreads();
-}
-
-// dst[n^3] (global) = the integration to n points of src[nc^3] (LDS)
-__device__ __forceinline__ void conv_restrict(int n, int nc,
-		const double *__restrict__ sp, const double *__restrict__ src,
-		double *__restrict__ dst, double *__restrict__ scr)
-{
-	double *t1 = scr, *t2 = scr + nc * nc * n;
-	for (int q = threadIdx.x; q < nc * nc * n; q += blockDim.x) {
-		const int p = q % n, kj = q / n;
-		double s = 0.0;
-		for (int c = 0; c < nc; ++c)
-			s += sp[p * nc + c] * src[kj * nc + c];
-		t1[q] = s;
-	}
-	__syncthreads();
-	for (int q = threadIdx.x; q < nc * n * n; q += blockDim.x) {
-		const int i = q % n, jq = (q / n) % n, k = q / (n * n);
-		double s = 0.0;
-		for (int l = 0; l < nc; ++l)
-			s += t1[(k * nc + l) * n + i] * sp[jq * nc + l];
-		t2[q] = s;
-	}
-	__syncthreads();
-	for (int q = threadIdx.x; q < n * n * n; q += blockDim.x) {
-		const int ji = q % (n * n), k = q / (n * n);
-		double s = 0.0;
-		for (int l = 0; l < nc; ++l)
-			s += t2[l * n * n + ji] * sp[k * nc + l];
-		dst[q] = s;
-	}
-	__syncthreads();
-}
-
-#define CONV_PTS 4                  // nc^3 / 1024 rounded up (nc <= 15)
-
-// the skew-symmetric operator at node r of the element (k_ns_conv_elem's
-// arithmetic): su the three u components, sv v_c, sd D, all at nc points
-__device__ __forceinline__ double conv_point(int nc, int r,
-		const double *__restrict__ su, const double *__restrict__ sv,
-		const double *__restrict__ sd, const P9 &ti,
-		const double *__restrict__ mass, long long q)
-{
-	const int c2 = nc * nc, c3 = c2 * nc;
-	const int i = r % nc, j = (r / nc) % nc, k = r / c2;
-	double jv[3] = { 0.0, 0.0, 0.0 };
-	double tb[3] = { 0.0, 0.0, 0.0 };
-	const double *rx = sv + (k * nc + j) * nc;
-	const double *ry = sv + k * c2 + i;
-	const double *rz = sv + j * nc + i;
-	const double *ux = su + (k * nc + j) * nc;
-	const double *uy = su + c3 + k * c2 + i;
-	const double *uz = su + 2 * c3 + j * nc + i;
-	for (int l = 0; l < nc; ++l) {
-		jv[0] += sd[i * nc + l] * rx[l];
-		jv[1] += sd[j * nc + l] * ry[l * nc];
-		jv[2] += sd[k * nc + l] * rz[l * c2];
-		tb[0] += sd[i * nc + l] * (ux[l] * rx[l]);
-		tb[1] += sd[j * nc + l] * (uy[l * nc] * ry[l * nc]);
-		tb[2] += sd[k * nc + l] * (uz[l * c2] * rz[l * c2]);
-	}
-	double tv[9];
-#pragma unroll
-	for (int a = 0; a < 9; ++a)
-		tv[a] = ti.p[a][q];
-	const double wj = mass[q];
-	double cv = 0.0;
-#pragma unroll
-	for (int a = 0; a < 3; ++a) {
-		double dv = 0.0;
+	// the factors at those nodes, issued after u's own loads and in flight
+	// during the other two contractions (the barriers order LDS only)
+	double gv[3][4][3];
+	const double *g = geo + e * 9 * C3;
+	interpolate(u, [&]() {
 #pragma unroll
 		for (int b = 0; b < 3; ++b) {
-			const double t = tv[3 * a + b] * jv[b];
-			dv = b == 0 ? t : t + dv;
-		}
-		const double t = su[a * c3 + r] * dv;
-		cv = a == 0 ? t : t + cv;
-	}
-	cv = cv * wj;
-	double cs = 0.0;
+			const Line w = line();
 #pragma unroll
-	for (int a = 0; a < 3; ++a) {
-		double d = 0.0;
+			for (int r = 0; r < 4; ++r) {
+				int zy, x;
+				result(w, b, r, zy, x);
+				// uniform base, 32-bit lane offset
+				const unsigned q = 8u * (unsigned) (zy * NC + x);
 #pragma unroll
-		for (int b = 0; b < 3; ++b) {
-			const double t = tv[3 * a + b] * tb[b];
-			d = b == 0 ? t : t + d;
+				for (int a = 0; a < 3; ++a)
+					gv[b][r][a] = *(const double *) ((const char *)
+							(g + (3 * a + b) * C3) + q);
+			}
 		}
-		cs = a == 0 ? d : cs + d;
+	});
+	// C_b, T_b at this lane's results, and u_b at its operands
+	double cc[3][4], tt[3][4], uo[3][SC];
+#pragma unroll
+	for (int b = 0; b < 3; ++b) {
+		const Line w = line();
+#pragma unroll
+		for (int r = 0; r < 4; ++r) {
+			int zy, x;
+			result(w, b, r, zy, x);
+			const double *q = ra + zy * KC + x;
+			tt[b][r] = (gv[b][r][0] + gv[b][r][1]) + gv[b][r][2];
+			cc[b][r] = q[0] * gv[b][r][0] + q[F3] * gv[b][r][1]
+				+ q[2 * F3] * gv[b][r][2];
+			// formed here: sunk to their use, their operands spilled
+			asm volatile("" : "+v"(tt[b][r]), "+v"(cc[b][r]));
+		}
 	}
-	cs = cs * wj;
-	return 0.5 * cs + 0.5 * cv;
-}
+	// operand k of line c along each direction (clamped: a[k >= NC] is 0
+	// and the value there is replaced by 0)
+	auto opnd = [&](const double *f, const Line &w, int b, int s) {
+		const int k = 4 * s + w.kq, kk = k < NC ? k : NC - 1;
+		const double x = b == 0 ? f[w.c * KC + kk]
+			: b == 1 ? f[(w.cz * NC + kk) * KC + w.ci]
+			: f[(kk * NC + w.cz) * KC + w.ci];
+		return k < NC ? x : 0.0;
+	};
+#pragma unroll
+	for (int b = 0; b < 3; ++b) {
+		const Line w = line();
+#pragma unroll
+		for (int s = 0; s < SC; ++s)
+			uo[b][s] = opnd(ra + b * F3, w, b, s);
+	}
+#pragma unroll
+	for (int b = 0; b < 3; ++b)
+#pragma unroll
+		for (int s = 0; s < SC; ++s)
+			asm volatile("" : "+v"(uo[b][s]));
+	lds_sync();
 
-__global__ void __launch_bounds__(1024)
-k_ns_conv_full(int n, int nc, const double *__restrict__ prol,
-		const double *__restrict__ dm, P3 u, P3 v, P9 ti,
-		const double *__restrict__ mass, M3 out)
-{
-	extern __shared__ double sm[];
-	const int c2 = nc * nc, c3 = c2 * nc, n3 = n * n * n;
-	double *sp = sm;                    // n*nc
-	double *sd = sp + n * nc;           // nc^2
-	double *su = sd + c2;               // u_0, u_1, u_2 at nc
-	double *sv = su + 3 * c3;           // v_c at nc, then the result
-	double *scr = sv + c3;              // transfer scratch
-	const long long e = blockIdx.x;
-	for (int q = threadIdx.x; q < n * nc; q += blockDim.x)
-		sp[q] = prol[q];
-	for (int q = threadIdx.x; q < c2; q += blockDim.x)
-		sd[q] = dm[q];
-	__syncthreads();
-	for (int a = 0; a < 3; ++a)
-		conv_prolong(n, nc, sp, u.p[a] + e * n3, su + a * c3, scr);
-	const long long b0 = e * c3;
-	for (int c = 0; c < 3; ++c) {
-		conv_prolong(n, nc, sp, v.p[c] + e * n3, sv, scr);
-		// this lane's nodes r = threadIdx.x + 1024 m, results in named
-		// registers (no array indexed by m)
-		double r0 = 0.0, r1 = 0.0, r2 = 0.0, r3 = 0.0;
+	interpolate(v, []() {});
+	// the operator at NC points in rb, direction by direction
+	double ad[SC];
+#pragma unroll
+	for (int s = 0; s < SC; ++s) {
+		const int k = 4 * s + kq;
+		const bool ok = col < NC && k < NC;
+		const double x = dm[ok ? col * NC + k : 0];
+		ad[s] = ok ? x : 0.0;
+	}
+#pragma unroll
+	for (int b = 0; b < 3; ++b) {
+		__builtin_amdgcn_sched_barrier(0);
+		const Line w = line();
+		const int kq = w.kq;
 #pragma unroll 1
-		for (int m = 0; m < CONV_PTS; ++m) {
-			const int r = threadIdx.x + m * 1024;
-			if (r >= c3)
-				break;
-			const double val = conv_point(nc, r, su, sv, sd, ti, mass, b0 + r);
-			r0 = m == 0 ? val : r0;
-			r1 = m == 1 ? val : r1;
-			r2 = m == 2 ? val : r2;
-			r3 = m == 3 ? val : r3;
-		}
-		__syncthreads();                // every read of sv is done
+		for (int f = 0; f < 3; ++f) {
+			conv_v4 d1 = { 0.0, 0.0, 0.0, 0.0 }, d2 = { 0.0, 0.0, 0.0, 0.0 };
 #pragma unroll
-		for (int m = 0; m < CONV_PTS; ++m) {
-			const int r = threadIdx.x + m * 1024;
-			if (r < c3)
-				sv[r] = m == 0 ? r0 : m == 1 ? r1 : m == 2 ? r2 : r3;
+			for (int s = 0; s < SC; ++s) {
+				const double x = opnd(ra + f * F3, w, b, s);
+				const double y = uo[b][s] * x;
+				if (b == 0) {
+					d1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x, ad[s], d1,
+							0, 0, 0);
+					d2 = __builtin_amdgcn_mfma_f64_16x16x4f64(y, ad[s], d2,
+							0, 0, 0);
+				} else {
+					d1 = __builtin_amdgcn_mfma_f64_16x16x4f64(ad[s], x, d1,
+							0, 0, 0);
+					d2 = __builtin_amdgcn_mfma_f64_16x16x4f64(ad[s], y, d2,
+							0, 0, 0);
+				}
+			}
+#pragma unroll
+			for (int r = 0; r < 4; ++r) {
+				const int m = CONV_ROW(r);
+				const double x = cc[b][r] * d1[r] + tt[b][r] * d2[r];
+				if (b == 0) {
+					const int l = 16 * wave + m;
+					if (l < C2 && w.col < NC)
+						rb[f * F3 + l * KC + w.col] = x;
+				} else if (w.ok && m < NC) {
+					double *o = rb + f * F3 + (b == 1
+						? (w.cz * NC + m) * KC + w.ci
+						: (m * NC + w.cz) * KC + w.ci);
+					*o = b == 1 ? *o + x : 0.5 * (*o + x);
+				}
+			}
 		}
-		__syncthreads();
-		conv_restrict(n, nc, sp, sv, out.p[c] + e * n3, scr);
+		lds_sync();
 	}
+	// integrated back to N points (the transposed contractions)
+	double ar[SC];
+#pragma unroll
+	for (int s = 0; s < SC; ++s) {
+		const int k = 4 * s + kq;
+		const bool ok = col < N && k < NC;
+		const double x = prol[ok ? col * NC + k : 0];
+		ar[s] = ok ? x : 0.0;
+	}
+	// ([p][z][y], [q][p][z], then z, y, x in global memory)
+	conv_stage<N, NC, C2, NC * KC, W, true>(ar, wave, lane, dump,
+		[&](int f, int l) { return rb + f * F3 + l * KC; },
+		[&](int f, int l) {
+			return ra + f * (N * NC * KC) + (l / NC) * KC + l % NC;
+		});
+	lds_sync();
+	conv_stage<N, NC, N * NC, N * KC, W, true>(ar, wave, lane, dump,
+		[&](int f, int l) { return ra + f * (N * NC * KC) + l * KC; },
+		[&](int f, int l) {
+			return rb + f * (N2 * KC) + (l / NC) * KC + l % NC;
+		});
+	lds_sync();
+	double *o0 = out.p[0] + e * N3, *o1 = out.p[1] + e * N3,
+		*o2 = out.p[2] + e * N3;
+	conv_stage<N, NC, N2, N2, W, false>(ar, wave, lane, nullptr,
+		[&](int f, int l) { return rb + f * (N2 * KC) + l * KC; },
+		[&](int f, int l) { return (f == 0 ? o0 : f == 1 ? o1 : o2) + l; });
+}
+
+template <int N>
+static int launch_conv(hipStream_t st, int nel, const double *prol,
+		const double *dm, const P3 &u, const P3 &v, const double *geo,
+		const M3 &out)
+{
+	constexpr int NC = (3 * N) / 2;
+	using S = ConvShape<N, NC>;
+	static_assert(S::W <= 16 && S::BYTES <= 160 * 1024, "element too large");
+	if (hipFuncSetAttribute((const void *) k_ns_conv<N, NC>,
+			hipFuncAttributeMaxDynamicSharedMemorySize, (int) S::BYTES)
+			!= hipSuccess) {
+		ssx_set_error("k_ns_conv: %zu bytes of LDS refused", S::BYTES);
+		return SSX_EHIP;
+	}
+	hipLaunchKernelGGL((k_ns_conv<N, NC>), dim3(nel), dim3(64 * S::W),
+			S::BYTES, st, prol, dm, u, v, geo, out);
+	return SSX_OK;
 }
 
 // f += (w_b w_a) n_s g on the face nodes of every face s of an element
@@ -646,86 +679,28 @@ extern "C" int ssxk_ns_grad(void *st, size_t nt, int n, const double *dm,
 	return SSX_OK;
 }
 
-extern "C" int ssxk_ns_conv(void *st, size_t nt, int n, const double *dm,
-		const double *const u[3], const double *const v[3],
-		const double *const Jv[9], const double *const ti[9],
-		const double *mass, double *const out[3])
+// geo: [nel][9][nc^3], component 3a+b w detJ d xi_b / d x_a at the nc =
+// 3n/2 points; n in [2, 10]
+extern "C" int ssxk_ns_conv(void *stream, int nel, int n, const double *prol,
+		const double *dm, const double *const u[3], const double *const v[3],
+		const double *geo, double *const out[3])
 {
-	P3 pu = { { u[0], u[1], u[2] } }, pv = { { v[0], v[1], v[2] } };
-	P9 pj, pt;
-	for (int k = 0; k < 9; ++k) {
-		pj.p[k] = Jv[k];
-		pt.p[k] = ti[k];
+	hipStream_t st = (hipStream_t) stream;
+	const P3 pu = { { u[0], u[1], u[2] } }, pv = { { v[0], v[1], v[2] } };
+	const M3 po = { { out[0], out[1], out[2] } };
+	int rc;
+	switch (n) {
+#define CASE(NN) case NN: rc = launch_conv<NN>(st, nel, prol, dm, pu, pv, \
+			geo, po); break;
+	CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(9) CASE(10)
+#undef CASE
+	default:
+		ssx_set_error("k_ns_conv: n = %d unsupported", n);
+		return SSX_EINVAL;
 	}
-	M3 po = { { out[0], out[1], out[2] } };
-	hipLaunchKernelGGL(k_ns_conv, dim3(ns_blocks(nt)), dim3(256), 0,
-			(hipStream_t) st, (long long) nt, n, dm, pu, pv, pj, pt, mass,
-			po);
+	if (rc != SSX_OK)
+		return rc;
 	NS_LAUNCH("k_ns_conv");
-	return SSX_OK;
-}
-
-extern "C" int ssxk_ns_conv_elem(void *st, int nel, int n, const double *dm,
-		const double *const u[3], const double *const v[3],
-		const double *const ti[9], const double *mass, double *const out[3])
-{
-	const size_t bytes = sizeof(double) * (4 * (size_t) n * n * n
-			+ (size_t) n * n);
-	if (n < 2 || bytes > 160 * 1024) {
-		ssx_set_error("k_ns_conv_elem: n = %d does not fit LDS", n);
-		return SSX_EINVAL;
-	}
-	P3 pu = { { u[0], u[1], u[2] } }, pv = { { v[0], v[1], v[2] } };
-	P9 pt;
-	for (int k = 0; k < 9; ++k)
-		pt.p[k] = ti[k];
-	M3 po = { { out[0], out[1], out[2] } };
-	if (hipFuncSetAttribute((const void *) k_ns_conv_elem,
-			hipFuncAttributeMaxDynamicSharedMemorySize, (int) bytes)
-			!= hipSuccess) {
-		ssx_set_error("k_ns_conv_elem: %zu bytes of LDS refused", bytes);
-		return SSX_EHIP;
-	}
-	hipLaunchKernelGGL(k_ns_conv_elem, dim3(nel), dim3(1024), bytes,
-			(hipStream_t) st, n, dm, pu, pv, pt, mass, po);
-	NS_LAUNCH("k_ns_conv_elem");
-	return SSX_OK;
-}
-
-// LDS of k_ns_conv_full, bytes
-extern "C" size_t ssxk_ns_conv_full_bytes(int n, int nc)
-{
-	const size_t scr_p = CONV_SCR((size_t) n, (size_t) nc);
-	const size_t scr_r = (size_t) nc * nc * n + (size_t) nc * n * n;
-	return sizeof(double) * ((size_t) n * nc + (size_t) nc * nc
-			+ 4 * (size_t) nc * nc * nc + (scr_p > scr_r ? scr_p : scr_r));
-}
-
-extern "C" int ssxk_ns_conv_full(void *st, int nel, int n, int nc,
-		const double *prol, const double *dm, const double *const u[3],
-		const double *const v[3], const double *const ti[9],
-		const double *mass, double *const out[3])
-{
-	const size_t bytes = ssxk_ns_conv_full_bytes(n, nc);
-	if (n < 2 || nc < n || nc * nc * nc > CONV_PTS * 1024
-			|| bytes > 160 * 1024) {
-		ssx_set_error("k_ns_conv_full: n = %d, nc = %d unsupported", n, nc);
-		return SSX_EINVAL;
-	}
-	P3 pu = { { u[0], u[1], u[2] } }, pv = { { v[0], v[1], v[2] } };
-	P9 pt;
-	for (int k = 0; k < 9; ++k)
-		pt.p[k] = ti[k];
-	M3 po = { { out[0], out[1], out[2] } };
-	if (hipFuncSetAttribute((const void *) k_ns_conv_full,
-			hipFuncAttributeMaxDynamicSharedMemorySize, (int) bytes)
-			!= hipSuccess) {
-		ssx_set_error("k_ns_conv_full: %zu bytes of LDS refused", bytes);
-		return SSX_EHIP;
-	}
-	hipLaunchKernelGGL(k_ns_conv_full, dim3(nel), dim3(1024), bytes,
-			(hipStream_t) st, n, nc, prol, dm, pu, pv, pt, mass, po);
-	NS_LAUNCH("k_ns_conv_full");
 	return SSX_OK;
 }
 
