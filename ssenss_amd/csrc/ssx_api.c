@@ -489,9 +489,12 @@ int ssx_create(ssx_ctx **out, const ssx_mesh *m)
 		const size_t nt = c->lev[0].ntot;
 		size_t np = (size_t) 12 * SSX_NPART;   /* FCG: 10 dots at once */
 		for (int l = 0; l < nl; ++l) {
-			/* one operator partial per element, then DSS partials */
+			/* one operator partial per element, then DSS partials or the
+			 * update's (its own range: replayed reductions read one kind
+			 * while the other is written) */
+			const size_t nd = (size_t) ssxk_dss_blocks(c->lev[l].ngrp);
 			size_t q = (size_t) c->nel
-				+ (size_t) ssxk_dss_blocks(c->lev[l].ngrp);
+				+ (nd > 4 * SSX_NPART ? nd : 4 * SSX_NPART);
 			if (q > np)
 				np = q;
 		}
@@ -999,6 +1002,10 @@ int ssx_cg_start(ssx_ctx *c, int l, int op, int var, double *f,
 	return SSX_OK;
 }
 
+/* the slot of <r,z>_w after iteration k of a run of replayed iterations
+ * (k = -1: before the first; ssx_replay) */
+#define RDZ_SLOT(k) ((k) < 0 || (k) % 2 == 0 ? CG_RDZ : CG_RDZ1)
+
 /*
  * The same iteration fused: Ax (from the second iteration on with the
  * direction update p = (z - c) + beta p of the previous one) and the sum of
@@ -1073,10 +1080,21 @@ static int cg_level_fused(ssx_ctx *c, int l, int op, int var, double *f,
 	/* the solution step u += alpha p of each iteration is taken by the
 	 * next operator launch, from its load of p; the last one by a flush */
 	const int defer = !c->fused_red;
+	/* the two reductions of an iteration replayed by the kernels that need
+	 * them (two launches an iteration); the chunk's last one is a launch */
+	const int gather = c->gather_upd && L->gP > 0 && !c->fused_red;
+	const int replay = gather && c->nel <= SSX_REPLAY_NEL;
+	double *pu = replay ? c->part + c->nel : c->part;
+	const int nbu = gather ? ssxk_cg_update_blocks(nt) : 0;
 	for (;;) {
 		if (chunk > max_iter - launched)
 			chunk = max_iter - launched;
 		for (int k = 0; k < chunk; ++k) {
+			const ssx_replay rb = { pu, nbu, c->scal, o, RDZ_SLOT(k - 1),
+				RDZ_SLOT(k), launched + k, max_iter, pres, flags, eps_dev,
+				(double) L->nunique };
+			const ssx_replay ra = { c->part, c->nel, c->scal, o, RDZ_SLOT(k),
+				0, 0, 0, 0, NULL, 0.0, 0.0 };
 			/* from the second iteration on, the operator kernel first forms
 			 * p = (z - c) + beta p (solver.c:70-72) */
 			if (launched + k == 0)
@@ -1088,7 +1106,8 @@ static int cg_level_fused(ssx_ctx *c, int l, int op, int var, double *f,
 						c->scal,
 						o + CG_BETA, pres ? o + CG_NULLC : -1, ap, L->gf,
 						L->mass, L->dmat, c->lambda, L->bc, !pres, flags,
-						c->part, defer ? u : NULL, o + CG_ALPHA));
+						c->part, defer ? u : NULL, o + CG_ALPHA,
+						replay && k > 0 ? &rb : NULL));
 			if (c->fused_red && nbd > 0) {
 				TRY(ssxk_dss_all_red(st, L->grp, L->ngrp, ap, NULL, NULL,
 						flags, &lr0));
@@ -1099,11 +1118,13 @@ static int cg_level_fused(ssx_ctx *c, int l, int op, int var, double *f,
 			if (c->gather_upd && L->gP > 0) {
 				/* alpha needs only the operator's partials; the
 				 * update then assembles Ap as it reads it */
-				TRY(ssxk_cg_reduce(st, 0, c->part, nba, c->scal, o, flags,
-						eps_dev, max_iter, L->nunique, pres));
+				if (!replay)
+					TRY(ssxk_cg_reduce(st, 0, c->part, nba, c->scal, o, flags,
+							eps_dev, max_iter, L->nunique, pres));
 				TRY(ssxk_cg_update_g(st, nt, L->n3, L->gP, L->gsoff,
 						L->gtab, c->scal, o + CG_ALPHA, p, ap,
-						defer ? NULL : u, r, z, dinv, pres, c->part, flags));
+						defer ? NULL : u, r, z, dinv, pres, pu, flags,
+						replay ? &ra : NULL));
 			} else {
 				TRY(ssxk_dss_all(st, L->grp, L->ngrp, ap, NULL, NULL, 0,
 						flags));
@@ -1113,8 +1134,10 @@ static int cg_level_fused(ssx_ctx *c, int l, int op, int var, double *f,
 						defer ? NULL : u, r, z, dinv, L->scale, pres, c->part,
 						flags));
 			}
-			TRY(ssxk_cg_reduce(st, 1, c->part, 0, c->scal, o, flags,
-					eps_dev, max_iter, L->nunique, pres));
+			if (!replay || k == chunk - 1)
+				TRY(ssxk_cg_reduce1(st, pu, nbu, c->scal, o,
+						replay ? RDZ_SLOT(k) : CG_RDZ, flags, eps_dev,
+						max_iter, L->nunique, pres));
 		}
 		launched += chunk;
 		hipStream_t hs = (hipStream_t) st;
@@ -1365,7 +1388,18 @@ static int cg_level_lp(ssx_ctx *c, int l, int op, int var, float *f,
 	 * with the operator's loads pipelined: FP32 0.193 -> 0.197 s, BF16
 	 * factors 0.183 -> 0.185 s, bit-identical results) */
 	const int defer = 0;
+	/* as cg_level_fused: reductions replayed on small levels */
+	const int gather = c->gather_upd && L->gP > 0
+		&& !(c->fused_red && ssxk_dss_blocks(L->ngrp) > 0);
+	const int replay = gather && c->nel <= SSX_REPLAY_NEL_LP;
+	double *pu = replay ? c->part + c->nel : c->part;
+	const int nbu = gather ? ssxk_cg_update_blocks(nt) : 0;
 	for (int k = 0; k < max_iter; ++k) {
+		const ssx_replay rb = { pu, nbu, c->scal, o, RDZ_SLOT(k - 1),
+			RDZ_SLOT(k), k, max_iter, pres, flags, eps,
+			(double) L->nunique };
+		const ssx_replay ra = { c->part, c->nel, c->scal, o, RDZ_SLOT(k), 0,
+			0, 0, 0, NULL, 0.0, 0.0 };
 		if (k == 0)
 			TRY(ssxk_ax_lp(st, L->lp_prec, L->n, L->axv[L->lp_prec], c->nel,
 					op, p, ap, L->gf_lp,
@@ -1376,7 +1410,8 @@ static int cg_level_lp(ssx_ctx *c, int l, int op, int var, float *f,
 					c->nel, op, z, p,
 					c->scal, o + CG_BETA, pres ? o + CG_NULLC : -1, ap,
 					L->gf_lp, L->mass_lp, L->dmat_lp, c->lambda, L->bc, !pres,
-					flags, c->part, defer ? u : NULL, o + CG_ALPHA));
+					flags, c->part, defer ? u : NULL, o + CG_ALPHA,
+					replay ? &rb : NULL));
 		if (c->fused_red && ssxk_dss_blocks(L->ngrp) > 0) {
 			const ssx_lastred lr0 = { c->redctr, c->part, nba, c->scal, o,
 				max_iter, pres, flags, eps, (double) L->nunique };
@@ -1389,11 +1424,12 @@ static int cg_level_lp(ssx_ctx *c, int l, int op, int var, float *f,
 			continue;
 		}
 		if (c->gather_upd && L->gP > 0) {
-			TRY(ssxk_cg_reduce(st, 0, c->part, nba, c->scal, o, flags, eps,
-					max_iter, L->nunique, pres));
+			if (!replay)
+				TRY(ssxk_cg_reduce(st, 0, c->part, nba, c->scal, o, flags,
+						eps, max_iter, L->nunique, pres));
 			TRY(ssxk_cg_update_g_lp(st, nt, L->n3, L->gP, L->gsoff, L->gtab,
 					c->scal, o + CG_ALPHA, p, ap, defer ? NULL : u, r, z,
-					dinv, pres, c->part, flags));
+					dinv, pres, pu, flags, replay ? &ra : NULL));
 		} else {
 			TRY(ssxk_dss_all_lp(st, L->grp, L->ngrp, ap, NULL, NULL, 0,
 					flags));
@@ -1403,8 +1439,10 @@ static int cg_level_lp(ssx_ctx *c, int l, int op, int var, float *f,
 					defer ? NULL : u, r, z, dinv, L->scale_lp, pres, c->part,
 					flags));
 		}
-		TRY(ssxk_cg_reduce(st, 1, c->part, 0, c->scal, o, flags, eps,
-				max_iter, L->nunique, pres));
+		if (!replay || k == max_iter - 1)
+			TRY(ssxk_cg_reduce1(st, pu, nbu, c->scal, o,
+					replay ? RDZ_SLOT(k) : CG_RDZ, flags, eps, max_iter,
+					L->nunique, pres));
 	}
 	if (defer && max_iter > 0)
 		TRY(ssxk_cg_uflush_lp(st, nt, c->scal, o + CG_ALPHA, p, u));

@@ -67,24 +67,124 @@ struct PUpd {
 	int ib, ic;
 	void *u;                     // nullable: u += scal[ia] p_old first
 	int ia;
+	ssx_replay rp;               // rp.part: scalars replayed, not read
 };
+
+// largest launch that reads the done flag along with its operands (a launch
+// of a stopped solve then loads one element a workgroup for nothing)
+#define SSX_LATE_FLAG_GRID 2048
+
+// the scalars of the fused direction update
+struct AxScal {
+	double b, c, a;              // beta, null-space constant, alpha
+	bool stop;                   // the solve has stopped: nothing to do
+};
+
+// Sums of the nq quantities (SSX_NPART apart) of m <= SSX_NPART partials in
+// exactly the order of a 1024-lane k_cg_reduce, by the workgroup's first
+// L lanes (64, or 32 where the workgroup is smaller than a wavefront): lane l
+// holds virtual lanes l, l + L, ..., folded as the tree's levels above L
+// do, the levels below by shuffles.  Lane 0 returns the sums.
+template <int L>
+__device__ __forceinline__ void replay_sums(const double *__restrict__ part,
+		int m, int nq, double out[4])
+{
+	constexpr int R = 1024 / L;
+	const int l = threadIdx.x;
+#pragma unroll
+	for (int c = 0; c < 4; ++c) {
+		out[c] = 0.0;
+		if (c >= nq)
+			break;
+		double v[R];
+#pragma unroll
+		for (int i = 0; i < R; ++i) {
+			// branch-free: an unused slot loads part[0] and discards it
+			const int q = l + L * i;
+			const double t = part[q < m ? c * SSX_NPART + q : 0];
+			v[i] = q < m ? t : 0.0;
+		}
+#pragma unroll
+		for (int st = R / 2; st > 0; st >>= 1)
+#pragma unroll
+			for (int i = 0; i < st; ++i)
+				v[i] += v[i + st];
+		out[c] = v[0];
+	}
+#pragma unroll
+	for (int st = L / 2; st > 0; st >>= 1)
+#pragma unroll
+		for (int c = 0; c < 4; ++c)
+			out[c] += __shfl_down(out[c], st, L);
+}
+
+// beta, the null-space constant and the stopping test of the previous
+// iteration (cg_scalars1) formed by every workgroup from the update's
+// partials; workgroup 0 stores them.  Every lane of the workgroup calls it;
+// dn: the solve had stopped before this launch (nothing is stored).
+template <int BLOCK>
+__device__ __forceinline__ AxScal replay_beta(const ssx_replay &rp, int dn)
+{
+	static_assert(BLOCK >= 32, "workgroup smaller than the replay's lanes");
+	constexpr int L = BLOCK >= 64 ? 64 : 32;
+	__shared__ double s_rp[3];
+	// loaded with the partials, not after them: another trip to memory
+	// costs a microsecond
+	const double old = rp.scal[rp.o + rp.rin];
+	const double tol = rp.eps >= 0.0 ? rp.eps : rp.scal[rp.o + CG_TOL];
+	if ((int) threadIdx.x < L) {
+		double v[4];
+		replay_sums<L>(rp.part, rp.cnt, rp.pressure ? 4 : 2, v);
+		if (threadIdx.x == 0) {
+			double c = 0.0, rz = v[0];
+			if (rp.pressure) {
+				c = v[2] / rp.nunique;
+				rz = rz - c * v[3];
+			}
+			const double beta = rz / old;
+			const bool stop = sqrt(v[1]) <= tol || rp.it >= rp.maxit
+				|| !(v[1] == v[1]);
+			if (blockIdx.x == 0 && !dn) {
+				rp.scal[rp.o + CG_NULLC] = c;
+				rp.scal[rp.o + CG_BETA] = beta;
+				rp.scal[rp.o + rp.rout] = rz;
+				rp.scal[rp.o + CG_RR] = v[1];
+				rp.flags[1] = rp.it;
+				if (stop)
+					rp.flags[0] = 1;
+			}
+			s_rp[0] = beta;
+			s_rp[1] = c;
+			s_rp[2] = stop || dn ? 1.0 : 0.0;
+		}
+	}
+	lds_sync();
+	AxScal s;
+	s.b = s_rp[0];
+	s.c = s_rp[1];
+	s.a = 0.0;
+	s.stop = s_rp[2] != 0.0;
+	return s;
+}
 
 // PUPD (PU >= 1): the update is done while the element is loaded, p is
 // written back and the operator is applied to the new p (the k_cg_pupdate
 // arithmetic); u is not read.  PU == 2: the previous iteration's solution
 // step uio += scal[ia] p_old is taken from the same load of p_old first
 // (the CG update then leaves u alone).
+// The scalars come from sc(), called by every lane once the element's loads
+// are out; hc: a null-space constant is subtracted.  Where sc says stop,
+// nothing is written.
 // One workgroup's elements [eblk*TEAMS, eblk*TEAMS + TEAMS): Au (masked)
 // written, and each lane's part of sum p (A_e p) over its nodes returned.
-template <int N, int OP, typename T, typename G, int PU, int V>
+template <int N, int OP, typename T, typename G, int PU, int V, typename SC>
 __device__ __forceinline__ double ax_team(int eblk, int nel,
 		const T *__restrict__ u, T *__restrict__ au,
 		const G *__restrict__ gf, const T *__restrict__ mass,
 		const T *__restrict__ dmat, T lambda,
 		const int *__restrict__ bc, int apply_mask,
-		const T *__restrict__ zin, T *__restrict__ pio,
-		const double *__restrict__ scal, int ib, int ic,
-		T *__restrict__ uio, int ia)
+		const T *__restrict__ zin, T *__restrict__ pio, T *__restrict__ uio,
+		bool hc, SC &&sc, bool *stopped)
 {
 	using S = AxShape<N, V>;
 	constexpr int N2 = S::N2, N3 = S::N3, P = S::P, TEAMS = S::TEAMS;
@@ -130,9 +230,6 @@ __device__ __forceinline__ double ax_team(int eblk, int nel,
 	const G *g = gf + (size_t) (act ? e : 0) * 6 * N3;
 	G fa[6], fb[6];
 	if (PU >= 1) {
-		const T bb = (T) scal[ib];
-		const T cc = ic >= 0 ? (T) -scal[ic] : T(0);
-		const T aa = PU == 2 ? (T) scal[ia] : T(0);
 		T po[N], zz[N], uo[PU == 2 ? N : 1];
 #pragma unroll
 		for (int k = 0; k < N; ++k) {
@@ -143,10 +240,17 @@ __device__ __forceinline__ double ax_team(int eblk, int nel,
 				uo[k] = uio[q];
 		}
 		ax_factors<NT, N3>(g, tid, fa);       // plane 0, in flight
+		const AxScal s = sc();
+		if (s.stop) {
+			*stopped = true;
+			return 0.0;
+		}
+		const T bb = (T) s.b, cc = hc ? (T) -s.c : T(0);
+		const T aa = PU == 2 ? (T) s.a : T(0);
 #pragma unroll
 		for (int k = 0; k < N; ++k) {
 			const size_t q = eoff + k * N2 + tid;
-			const T zv = ic >= 0 ? cc * T(1) + zz[k] : zz[k];
+			const T zv = hc ? cc * T(1) + zz[k] : zz[k];
 			T v = bb * po[k] + zv;
 			const bool m = mi || ((bits & 16) && k == 0)
 				|| ((bits & 32) && k == N - 1);
@@ -340,13 +444,33 @@ k_ax(int nel, const T *__restrict__ u, T *__restrict__ au,
 		const int *__restrict__ done, double *__restrict__ part,
 		const T *__restrict__ zin, T *__restrict__ pio,
 		const double *__restrict__ scal, int ib, int ic,
-		T *__restrict__ uio, int ia)
+		T *__restrict__ uio, int ia, ssx_replay rp)
 {
-	if (done && *done)          // solver already converged: no-op
+	// Solver already converged: no-op.  A small launch, which lasts a few
+	// trips to memory, reads the flag along with its operands instead of
+	// one trip ahead of them (PU: after the element's loads).
+	const bool late = PU >= 1 && gridDim.x <= SSX_LATE_FLAG_GRID;
+	const int dn = done ? *done : 0;
+	if (!late && dn)
 		return;
+	bool stopped = false;
 	const double pd = ax_team<N, OP, T, G, PU, V>(blockIdx.x, nel, u, au,
-			gf, mass, dmat, lambda, bc, apply_mask, zin, pio, scal, ib, ic,
-			uio, ia);
+			gf, mass, dmat, lambda, bc, apply_mask, zin, pio, uio, ic >= 0,
+			[&]() {
+				AxScal s;
+				const double al = PU == 2 ? scal[ia] : 0.0;
+				if (rp.part) {
+					s = replay_beta<AxShape<N, V>::BLOCK>(rp, dn);
+				} else {
+					s.b = scal[ib];
+					s.c = ic >= 0 ? scal[ic] : 0.0;
+					s.stop = dn != 0;
+				}
+				s.a = al;
+				return s;
+			}, &stopped);
+	if (stopped)
+		return;
 	if (part)
 		ax_elem_partial<N, V>(pd, part, blockIdx.x, nel);
 }
@@ -364,13 +488,13 @@ static void launch_ax1(hipStream_t st, int nel, int op, const void *u,
 				dim3(S::BLOCK), 0, st, nel, (const T *) u, (T *) au,
 				(const G *) gf, (const T *) mass, (const T *) dmat, (T) lambda,
 				bc, apply_mask, done, part, (const T *) pu.z, (T *) pu.p,
-				pu.scal, pu.ib, pu.ic, (T *) pu.u, pu.ia);
+				pu.scal, pu.ib, pu.ic, (T *) pu.u, pu.ia, pu.rp);
 	else
 		hipLaunchKernelGGL((k_ax<N, 0, T, G, PU, V>), dim3(grid),
 				dim3(S::BLOCK), 0, st, nel, (const T *) u, (T *) au,
 				(const G *) gf, (const T *) mass, (const T *) dmat, (T) lambda,
 				bc, apply_mask, done, part, (const T *) pu.z, (T *) pu.p,
-				pu.scal, pu.ib, pu.ic, (T *) pu.u, pu.ia);
+				pu.scal, pu.ib, pu.ic, (T *) pu.u, pu.ia, pu.rp);
 }
 
 template <int N, typename T, typename G, int V>
@@ -390,7 +514,7 @@ static void launch_ax_v(hipStream_t st, int nel, int op, const void *u,
 	else
 		launch_ax1<N, T, G, 0, V>(st, nel, op, u, au, gf, mass, dmat,
 				lambda, bc, apply_mask, done, part, PUpd{ nullptr, nullptr,
-				nullptr, 0, -1, nullptr, 0 });
+				nullptr, 0, -1, nullptr, 0, ssx_replay{} });
 }
 
 // dispatcher body shared by the per-precision files: n in [2,16], variant

@@ -41,11 +41,15 @@ k_bax(const ssx_bprob *__restrict__ pr, const ssx_bwork *__restrict__ tab)
 	// PUPD reads z and p and writes p; otherwise p is the operand
 	const double *u = PUPD ? nullptr : gptr(d->p);
 	double *pio = PUPD ? gptr(d->p) : nullptr;
+	bool stopped = false;
 	const double pd = ax_team<N, OP, double, double, PUPD ? 2 : 0, V>(
 			w.blk, d->nel,
 			u, gptr(d->ap), gptr(d->gf), gptr(d->mass), gptr(d->dmat),
 			d->lambda, gptr(d->bc), d->apply_mask, gptr(d->z), pio,
-			d->scal, CG_BETA, ic, PUPD ? gptr(d->u) : nullptr, CG_ALPHA);
+			PUPD ? gptr(d->u) : nullptr, ic >= 0, [&]() {
+				return AxScal{ d->scal[CG_BETA], ic >= 0 ? d->scal[ic] : 0.0,
+					d->scal[CG_ALPHA], false };
+			}, &stopped);
 	ax_elem_partial<N, V>(pd, d->part, w.blk, d->nel);
 }
 

@@ -31,11 +31,15 @@ k_bax_lp(const ssx_bprob *__restrict__ pr, const ssx_bwork *__restrict__ tab)
 	if (d->flags[0])
 		return;
 	const int ic = d->pressure ? CG_NULLC : -1;
+	bool stopped = false;
 	const double pd = ax_team<N, OP, float, G, 1, V>(w.blk, d->nel,
 			nullptr, gptr(d->ap_f), gptr((const G *) d->gf_lp),
 			gptr(d->mass_f), gptr(d->dmat_f), (float) d->lambda,
 			gptr(d->bc), d->apply_mask, gptr(d->z_f), gptr(d->p_f),
-			d->scal, CG_BETA, ic, nullptr, CG_ALPHA);
+			nullptr, ic >= 0, [&]() {
+				return AxScal{ d->scal[CG_BETA], ic >= 0 ? d->scal[ic] : 0.0,
+					0.0, false };
+			}, &stopped);
 	ax_elem_partial<N, V>(pd, d->part, w.blk, d->nel);
 }
 

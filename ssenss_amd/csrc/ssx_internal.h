@@ -308,21 +308,49 @@ int ssxk_ax(void *stream, int n, int v, int nel, int op, const double *u,
 		double *au, const double *gf, const double *mass,
 		const double *dmat, double lambda, const int *bc, int apply_mask,
 		const int *done, double *part);
+/* A reduction of the fused CG replayed by the kernel that needs it instead
+ * of a launch of its own (part != NULL): every workgroup sums the cnt
+ * partials exactly as ssxk_cg_reduce does and forms the same scalars;
+ * workgroup 0 stores them.  <r,z>_w alternates between the slots o + rin
+ * (read) and o + rout (written), so no workgroup reads a slot that another
+ * one of the launch writes; it: iterations completed before this launch. */
+typedef struct ssx_replay {
+	const double *part;
+	int cnt;                 /* <= SSX_NPART in ssxk_ax_pupd (mode 1)     */
+	double *scal;
+	int o, rin, rout, it, maxit, pressure;
+	int *flags;
+	double eps, nunique;
+} ssx_replay;
+/* Most elements of a level whose CG replays its reductions (FP64; FP32
+ * fields).  A replay costs the operator 3.6 us and the update 2.4 us where
+ * every workgroup has its slot at once, a launch 4.3 us and its gap.  The
+ * FP64 operator's registers leave 8 wavefronts a CU, so past about a
+ * thousand elements of two or more wavefronts the replay comes round
+ * after round.  Measured per CG iteration, launches / replayed: FP64 n = 8
+ * 64 elements 19.3 / 16.2 us, 1000: 26.6 / 25.3, 4096: 59.9 / 70.6, n = 12
+ * 216: 32.7 / 30.7, 1728: 114.5 / 119.1; FP32 V-cycle n = 8 64: 635 / 508
+ * us, 4096: 1169 / 1082, n = 12 1728: 1813 / 1776, n = 8 8000 (all
+ * replayed): 1646 / 1845. */
+#define SSX_REPLAY_NEL 1024
+#define SSX_REPLAY_NEL_LP 4096
 /* ssxk_ax of the new CG direction: p = (z - scal[ic]) + scal[ib] p
  * (ic < 0: no null-space constant), masked where apply_mask, written back
  * to p, and ap = A p -- the k_cg_pupdate of the previous iteration fused
  * into the operator; u (nullable): first u += scal[ia] p (old p), the
- * previous iteration's solution step */
+ * previous iteration's solution step; rp (nullable): beta, the null-space
+ * constant and the stopping test replayed from the update's partials
+ * (4 quantities, SSX_NPART apart; mode 1 of ssxk_cg_reduce) */
 int ssxk_ax_pupd(void *stream, int n, int v, int nel, int op, const double *z,
 		double *p, const double *scal, int ib, int ic, double *ap,
 		const double *gf, const double *mass, const double *dmat,
 		double lambda, const int *bc, int apply_mask, const int *done,
-		double *part, double *u, int ia);
+		double *part, double *u, int ia, const ssx_replay *rp);
 int ssxk_ax_pupd_lp(void *stream, int prec, int n, int v, int nel, int op,
 		const void *z, void *p, const double *scal, int ib, int ic, void *ap,
 		const void *gf, const void *mass, const void *dmat, double lambda,
 		const int *bc, int apply_mask, const int *done, double *part,
-		void *u, int ia);
+		void *u, int ia, const ssx_replay *rp);
 /* u += scal[ia] p whatever the done flags (the last solution step of a CG
  * whose steps the operator launches take: ssxk_ax_pupd with u, updates
  * with u = NULL) */
@@ -375,15 +403,19 @@ int ssxk_cg_update_red_lp(void *stream, size_t n, const double *scal, int ia,
 /* ssxk_cg_update with the DSS of ap as a gather over per-copy partner lists
  * (tab, soff from ssx_build_gather): ap is read unassembled and left so;
  * weights 1/M from the lists (no scale vector).  Bit-identical to
- * ssxk_dss_all followed by ssxk_cg_update. */
+ * ssxk_dss_all followed by ssxk_cg_update.  The workgroups, and so the
+ * partials of each quantity, are ssxk_cg_update_blocks(n) <= SSX_NPART; rp
+ * (nullable): alpha replayed from the operator's partials (mode 0). */
+int ssxk_cg_update_blocks(size_t n);
 int ssxk_cg_update_g(void *stream, size_t n, int n3, int P, const int *soff,
 		const int *tab, const double *scal, int ia, const double *p,
 		const double *ap, double *u, double *r, double *z, const double *dinv,
-		int pressure, double *part, const int *done);
+		int pressure, double *part, const int *done, const ssx_replay *rp);
 int ssxk_cg_update_g_lp(void *stream, size_t n, int n3, int P,
 		const int *soff, const int *tab, const double *scal, int ia,
 		const void *p, const void *ap, void *u, void *r, void *z,
-		const void *dinv, int pressure, double *part, const int *done);
+		const void *dinv, int pressure, double *part, const int *done,
+		const ssx_replay *rp);
 /* r = f - DSS(a) with the DSS of the unassembled a as a gather (lists as
  * ssxk_cg_update_g); init != 0: the CG start -- f = f * mask first (mask
  * nullable, f written back), then r, z = dinv r, p = z and the k_dot
@@ -413,6 +445,11 @@ int ssxk_cg_update_nb(void *stream, size_t n, const double *scal, int ia,
  * sums cnt partials per quantity (0: SSX_NPART) */
 int ssxk_cg_reduce(void *stream, int mode, const double *part, long long cnt,
 		double *scal, int o, int *flags, double eps, int maxit,
+		double nunique, int pressure);
+/* mode 1 with the old <r,z>_w in slot o + rin (after replayed iterations);
+ * the new one goes to o + CG_RDZ */
+int ssxk_cg_reduce1(void *stream, const double *part, long long cnt,
+		double *scal, int o, int rin, int *flags, double eps, int maxit,
 		double nunique, int pressure);
 /* scal[dst] = max(eps, rtol * sqrt(scal[src])) */
 int ssxk_cg_tol(void *stream, double *scal, int dst, int src, double eps,

@@ -84,9 +84,13 @@ extern "C" int ssxk_ax_pupd(void *stream, int n, int v, int nel, int op,
 		const double *z, double *p, const double *scal, int ib, int ic,
 		double *ap, const double *gf, const double *mass, const double *dmat,
 		double lambda, const int *bc, int apply_mask, const int *done,
-		double *part, double *u, int ia)
+		double *part, double *u, int ia, const ssx_replay *rp)
 {
-	const PUpd pu = { z, p, scal, ib, ic, u, ia };
+	if (rp && (rp->cnt < 1 || rp->cnt > SSX_NPART)) {
+		ssx_set_error("ssxk_ax_pupd: %d partials to replay", rp->cnt);
+		return SSX_EINVAL;
+	}
+	const PUpd pu = { z, p, scal, ib, ic, u, ia, rp ? *rp : ssx_replay{} };
 	return ssxk_ax_dispatch_f64(stream, n, v, nel, op, nullptr, ap, gf, mass,
 			dmat, lambda, bc, apply_mask, done, part, &pu);
 }
@@ -107,14 +111,18 @@ extern "C" int ssxk_ax_pupd_lp(void *stream, int prec, int n, int v, int nel,
 		int op, const void *z, void *p, const double *scal, int ib, int ic,
 		void *ap, const void *gf, const void *mass, const void *dmat,
 		double lambda, const int *bc, int apply_mask, const int *done,
-		double *part, void *u, int ia)
+		double *part, void *u, int ia, const ssx_replay *rp)
 {
+	if (rp && (rp->cnt < 1 || rp->cnt > SSX_NPART)) {
+		ssx_set_error("ssxk_ax_pupd_lp: %d partials to replay", rp->cnt);
+		return SSX_EINVAL;
+	}
 	if (u) {
 		ssx_set_error("ssxk_ax_pupd_lp: the deferred solution step is FP64 "
 				"only");
 		return SSX_EINVAL;
 	}
-	const PUpd pu = { z, p, scal, ib, ic, u, ia };
+	const PUpd pu = { z, p, scal, ib, ic, u, ia, rp ? *rp : ssx_replay{} };
 	if (prec == SSX_PREC_BF16)
 		return ssxk_ax_dispatch_bf16(stream, n, v, nel, op, nullptr, ap, gf,
 				mass, dmat, lambda, bc, apply_mask, done, part, &pu);
@@ -126,19 +134,20 @@ extern "C" int ssxk_ax_pupd_lp(void *stream, int prec, int n, int v, int nel,
 // CG scalar logic shared by k_cg_reduce and the last-workgroup reductions
 // ---------------------------------------------------------------------
 
-// mode 0: s[o+PAP] = pap; s[o+ALPHA] = s[o+RDZ] / pap
-__device__ __forceinline__ void cg_scalars0(double pap, double *scal, int o)
+// mode 0: s[o+PAP] = pap; s[o+ALPHA] = rdz / pap
+__device__ __forceinline__ void cg_scalars0(double pap, double rdz,
+		double *scal, int o)
 {
 	scal[o + CG_PAP] = pap;
-	scal[o + CG_ALPHA] = scal[o + CG_RDZ] / pap;
+	scal[o + CG_ALPHA] = rdz / pap;
 }
 
-// mode 1: null-space constant c = zs/nunique; rdz = rz - c rs;
-// beta = rdz / rdz_old; iteration count ++, done when sqrt(rr) <= eps
-// (eps < 0: s[o+TOL]) or count >= maxit or NaN
+// mode 1: null-space constant c = zs/nunique; rdz = rz - c rs; beta = rdz /
+// old; iteration count it0 + 1, done when sqrt(rr) <= tol or count >= maxit
+// or NaN
 __device__ __forceinline__ void cg_scalars1(double rz, double rr, double zs,
-		double rs, double *scal, int o, int *flags, double eps, int maxit,
-		double nunique, int pressure)
+		double rs, double old, int it0, double tol, double *scal, int o,
+		int *flags, int maxit, double nunique, int pressure)
 {
 	double c = 0.0;
 	if (pressure) {
@@ -146,12 +155,11 @@ __device__ __forceinline__ void cg_scalars1(double rz, double rr, double zs,
 		rz = rz - c * rs;
 	}
 	scal[o + CG_NULLC] = c;
-	scal[o + CG_BETA] = rz / scal[o + CG_RDZ];
+	scal[o + CG_BETA] = rz / old;
 	scal[o + CG_RDZ] = rz;
 	scal[o + CG_RR] = rr;
-	const int it = flags[1] + 1;
+	const int it = it0 + 1;
 	flags[1] = it;
-	const double tol = eps >= 0.0 ? eps : scal[o + CG_TOL];
 	if (sqrt(rr) <= tol || it >= maxit || !(rr == rr))
 		flags[0] = 1;
 }
@@ -254,7 +262,7 @@ k_dss_all(long long G2, long long G4, long long G8, const int *__restrict__ i2,
 		__shared__ double sr[256];
 		const double pap = sum_as_1024(lr.part, lr.cnt, sr);
 		if (threadIdx.x == 0)
-			cg_scalars0(pap, lr.scal, lr.o);
+			cg_scalars0(pap, lr.scal[lr.o + CG_RDZ], lr.scal, lr.o);
 	}
 }
 
@@ -401,9 +409,66 @@ k_cg_update(size_t n, const double *__restrict__ scal, int ia,
 			v[c] = sum_as_1024(lr.part + (size_t) c * SSX_NPART, SSX_NPART,
 					sh[0]);
 		if (threadIdx.x == 0)
-			cg_scalars1(v[0], v[1], v[2], v[3], lr.scal, lr.o, lr.flags,
-					lr.eps, lr.maxit, lr.nunique, lr.pressure);
+			cg_scalars1(v[0], v[1], v[2], v[3], lr.scal[lr.o + CG_RDZ],
+					lr.flags[1], lr.eps >= 0.0 ? lr.eps
+					: lr.scal[lr.o + CG_TOL], lr.scal, lr.o, lr.flags,
+					lr.maxit, lr.nunique, lr.pressure);
 	}
+}
+
+// alpha = <r,z>_w / sum of the operator's partials, formed by every
+// 256-lane workgroup in the order of a 1024-lane k_cg_reduce mode 0 (lane t
+// folds virtual lanes t, t+256, t+512, t+768 as the first two tree levels
+// do); workgroup 0 stores it.  sh: 256 doubles.
+__device__ double replay_alpha(const ssx_replay &rp, double *sh)
+{
+	const double rdz = rp.scal[rp.o + rp.rin];   // with the partials
+	double a[4];
+#pragma unroll
+	for (int v = 0; v < 4; ++v) {
+		// up to 4 of the virtual lane's partials in flight, added in order
+		double x[4];
+		const int q0 = threadIdx.x + 256 * v;
+#pragma unroll
+		for (int i = 0; i < 4; ++i) {
+			const int q = q0 + 1024 * i;
+			const double t = rp.part[q < rp.cnt ? q : 0];
+			x[i] = q < rp.cnt ? t : 0.0;
+		}
+		a[v] = x[0];
+#pragma unroll
+		for (int i = 1; i < 4; ++i)
+			if (q0 + 1024 * i < rp.cnt)
+				a[v] += x[i];
+		for (int q = q0 + 4096; q < rp.cnt; q += 1024)
+			a[v] += rp.part[q];
+	}
+	a[0] += a[2];
+	a[1] += a[3];
+	a[0] += a[1];
+	sh[threadIdx.x] = a[0];
+	lds_sync();
+	if (threadIdx.x < 128)
+		sh[threadIdx.x] += sh[threadIdx.x + 128];
+	lds_sync();
+	if (threadIdx.x < 64) {
+		double w = sh[threadIdx.x] + sh[threadIdx.x + 64];
+#pragma unroll
+		for (int st = 32; st > 0; st >>= 1)
+			w += __shfl_down(w, st, 64);
+		if (threadIdx.x == 0) {
+			const double al = rdz / w;
+			if (blockIdx.x == 0) {
+				rp.scal[rp.o + CG_PAP] = w;
+				rp.scal[rp.o + CG_ALPHA] = al;
+			}
+			sh[0] = al;
+		}
+	}
+	lds_sync();
+	const double al = sh[0];
+	lds_sync();
+	return al;
 }
 
 // k_cg_update with the DSS of Ap done as a gather: every copy adds its
@@ -416,25 +481,34 @@ k_cg_update(size_t n, const double *__restrict__ scal, int ia,
 // issues the table and partner loads of all U before using any: the
 // partner loads depend on the table loads, which depend on soff, and one
 // node at a time leaves those three round trips unoverlapped.
-template <typename T, int U, bool UPD>
+// RP: alpha is replayed from the operator's partials once the first nodes'
+// loads are out (cg_scalars0 in every workgroup), and a launch of at most
+// one trip a lane reads the done flag along with its operands.  A kernel of
+// its own: the same code behind a run-time test cost the plain launch 20 %.
+template <typename T, int U, bool UPD, bool RP>
 __global__ void __launch_bounds__(256)
 k_cg_update_g(unsigned n, unsigned n3, int P, const int *__restrict__ soff,
 		const int *__restrict__ tab, const double *__restrict__ scal, int ia,
 		const T *__restrict__ p, const T *__restrict__ ap,
 		T *__restrict__ u, T *__restrict__ r, T *__restrict__ z,
 		const T *__restrict__ dinv, int pressure,
-		double *__restrict__ part, const int *__restrict__ done)
+		double *__restrict__ part, const int *__restrict__ done,
+		ssx_replay rp)
 {
-	if (done && *done)
+	const bool late = RP && (size_t) gridDim.x * (256u * U) >= n;
+	const int dn = done ? *done : 0;
+	if (!late && dn)
 		return;
 	__shared__ double sh[4][256];
 	constexpr bool HOIST = sizeof(T) == 4;
-	const T a = (T) scal[ia];
+	bool have = !RP;
+	T a = RP ? T(0) : (T) scal[ia];
 	const unsigned stride = gridDim.x * 256u;
 	const unsigned lb = xcd_block();
 	double acc[4] = { 0.0, 0.0, 0.0, 0.0 };
-	for (unsigned q0 = lb * 256u + threadIdx.x; q0 < n;
-			q0 += U * stride) {
+	// RP: the trip count is the workgroup's (the replay has barriers)
+	for (unsigned q0 = lb * 256u + threadIdx.x;
+			(RP ? q0 - threadIdx.x : q0) < n; q0 += U * stride) {
 		int ix[U][7];
 		T own[U], pv[U][7], rq[U], dq[U], pq[U], uq[U];
 #pragma unroll
@@ -471,6 +545,12 @@ k_cg_update_g(unsigned n, unsigned n3, int P, const int *__restrict__ soff,
 #pragma unroll
 			for (int k = 0; k < 7; ++k)
 				pv[v][k] = ix[v][k] >= 0 ? ap[ix[v][k]] : T(0);
+		if (RP && dn)
+			return;
+		if (!have) {
+			a = (T) replay_alpha(rp, sh[0]);
+			have = true;
+		}
 #pragma unroll
 		for (int v = 0; v < U; ++v) {
 			const unsigned q = q0 + v * stride;
@@ -506,28 +586,41 @@ k_cg_update_g(unsigned n, unsigned n3, int P, const int *__restrict__ soff,
 		part[(size_t) threadIdx.x * SSX_NPART + lb] = sh[threadIdx.x][0];
 }
 
+// one workgroup a 256 nodes, at most SSX_NPART (the grid-stride order of a
+// larger grid leaves the same nodes to each)
+extern "C" int ssxk_cg_update_blocks(size_t n)
+{
+	const size_t b = (n + 255) / 256;
+	return b < 1 ? 1 : b < SSX_NPART ? (int) b : SSX_NPART;
+}
+
 template <typename T>
 static int launch_cg_update_g(hipStream_t st, size_t n, int n3, int P,
 		const int *soff, const int *tab, const double *scal, int ia,
 		const void *p, const void *ap, void *u, void *r, void *z,
-		const void *dinv, int pressure, double *part, const int *done)
+		const void *dinv, int pressure, double *part, const int *done,
+		const ssx_replay *rp)
 {
 	if (n >= (1ull << 31) || n % (size_t) n3) {
 		ssx_set_error("k_cg_update_g: %zu nodes, %d per element", n, n3);
 		return SSX_EINVAL;
 	}
-	if (u)
-		hipLaunchKernelGGL((k_cg_update_g<T, SSX_GATHER_U, true>),
-				dim3(SSX_NPART), dim3(256), 0, st, (unsigned) n,
-				(unsigned) n3, P, soff, tab, scal, ia, (const T *) p,
-				(const T *) ap, (T *) u, (T *) r, (T *) z, (const T *) dinv,
-				pressure, part, done);
+	const dim3 g(ssxk_cg_update_blocks(n));
+	const ssx_replay none = {};
+#define UPDATE_G(UU, RR) hipLaunchKernelGGL( \
+		(k_cg_update_g<T, SSX_GATHER_U, UU, RR>), g, dim3(256), 0, st, \
+		(unsigned) n, (unsigned) n3, P, soff, tab, scal, ia, \
+		(const T *) p, (const T *) ap, (T *) u, (T *) r, (T *) z, \
+		(const T *) dinv, pressure, part, done, rp ? *rp : none)
+	if (u && rp)
+		UPDATE_G(true, true);
+	else if (u)
+		UPDATE_G(true, false);
+	else if (rp)
+		UPDATE_G(false, true);
 	else
-		hipLaunchKernelGGL((k_cg_update_g<T, SSX_GATHER_U, false>),
-				dim3(SSX_NPART), dim3(256), 0, st, (unsigned) n,
-				(unsigned) n3, P, soff, tab, scal, ia, (const T *) p,
-				(const T *) ap, (T *) u, (T *) r, (T *) z, (const T *) dinv,
-				pressure, part, done);
+		UPDATE_G(false, false);
+#undef UPDATE_G
 	LAUNCH_CHECK("k_cg_update_g");
 	return SSX_OK;
 }
@@ -535,19 +628,21 @@ static int launch_cg_update_g(hipStream_t st, size_t n, int n3, int P,
 extern "C" int ssxk_cg_update_g(void *stream, size_t n, int n3, int P,
 		const int *soff, const int *tab, const double *scal, int ia,
 		const double *p, const double *ap, double *u, double *r, double *z,
-		const double *dinv, int pressure, double *part, const int *done)
+		const double *dinv, int pressure, double *part, const int *done,
+		const ssx_replay *rp)
 {
 	return launch_cg_update_g<double>((hipStream_t) stream, n, n3, P, soff,
-			tab, scal, ia, p, ap, u, r, z, dinv, pressure, part, done);
+			tab, scal, ia, p, ap, u, r, z, dinv, pressure, part, done, rp);
 }
 
 extern "C" int ssxk_cg_update_g_lp(void *stream, size_t n, int n3, int P,
 		const int *soff, const int *tab, const double *scal, int ia,
 		const void *p, const void *ap, void *u, void *r, void *z,
-		const void *dinv, int pressure, double *part, const int *done)
+		const void *dinv, int pressure, double *part, const int *done,
+		const ssx_replay *rp)
 {
 	return launch_cg_update_g<float>((hipStream_t) stream, n, n3, P, soff,
-			tab, scal, ia, p, ap, u, r, z, dinv, pressure, part, done);
+			tab, scal, ia, p, ap, u, r, z, dinv, pressure, part, done, rp);
 }
 
 __device__ __forceinline__ double block_sum256(double v, double *sh);
@@ -753,11 +848,14 @@ extern "C" int ssxk_cg_uflush_lp(void *stream, size_t n, const double *scal,
 
 __global__ void __launch_bounds__(1024)
 k_cg_reduce(int mode, const double *__restrict__ part, long long cnt,
-		double *__restrict__ scal, int o, int *__restrict__ flags,
+		double *__restrict__ scal, int o, int rin, int *__restrict__ flags,
 		double eps, int maxit, double nunique, int pressure)
 {
-	if (flags[0])
-		return;
+	// the flag and the old scalars are loaded with the partials: this launch
+	// lasts as long as its trips to memory
+	const int dn = flags[0], it0 = flags[1];
+	const double old = scal[o + rin];
+	const double tol = mode == 0 || eps >= 0.0 ? eps : scal[o + CG_TOL];
 	__shared__ double sh[4][1024];
 	const int nq = mode == 0 ? 1 : (pressure ? 4 : 2);
 	const long long m = (mode == 0 || cnt > 0) ? cnt : SSX_NPART;
@@ -773,6 +871,8 @@ k_cg_reduce(int mode, const double *__restrict__ part, long long cnt,
 		const double v = part[use ? (size_t) c * SSX_NPART + t : 0];
 		first[c] = use ? v : 0.0;
 	}
+	if (dn)
+		return;
 	for (int c = 0; c < 4; ++c) {
 		double acc = 0.0;
 		if (c < nq && t < m) {
@@ -814,10 +914,10 @@ k_cg_reduce(int mode, const double *__restrict__ part, long long cnt,
 	if (threadIdx.x != 0)
 		return;
 	if (mode == 0)
-		cg_scalars0(v[0], scal, o);
+		cg_scalars0(v[0], old, scal, o);
 	else
-		cg_scalars1(v[0], v[1], v[2], v[3], scal, o, flags, eps, maxit,
-				nunique, pressure);
+		cg_scalars1(v[0], v[1], v[2], v[3], old, it0, tol, scal, o, flags,
+				maxit, nunique, pressure);
 }
 
 __global__ void k_cg_tol(double *scal, int dst, int src, double eps,
@@ -947,8 +1047,19 @@ extern "C" int ssxk_cg_reduce(void *stream, int mode, const double *part,
 		int maxit, double nunique, int pressure)
 {
 	hipLaunchKernelGGL(k_cg_reduce, dim3(1), dim3(1024), 0,
-			(hipStream_t) stream, mode, part, cnt, scal, o, flags, eps, maxit,
-			nunique, pressure);
+			(hipStream_t) stream, mode, part, cnt, scal, o, (int) CG_RDZ, flags,
+			eps, maxit, nunique, pressure);
+	LAUNCH_CHECK("k_cg_reduce");
+	return SSX_OK;
+}
+
+extern "C" int ssxk_cg_reduce1(void *stream, const double *part,
+		long long cnt, double *scal, int o, int rin, int *flags, double eps,
+		int maxit, double nunique, int pressure)
+{
+	hipLaunchKernelGGL(k_cg_reduce, dim3(1), dim3(1024), 0,
+			(hipStream_t) stream, 1, part, cnt, scal, o, rin, flags, eps,
+			maxit, nunique, pressure);
 	LAUNCH_CHECK("k_cg_reduce");
 	return SSX_OK;
 }
