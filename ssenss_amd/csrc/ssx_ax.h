@@ -497,24 +497,48 @@ static void launch_ax1(hipStream_t st, int nel, int op, const void *u,
 				pu.scal, pu.ib, pu.ic, (T *) pu.u, pu.ia, pu.rp);
 }
 
+#include "ssx_axm.h"
+
 template <int N, typename T, typename G, int V>
 static void launch_ax_v(hipStream_t st, int nel, int op, const void *u,
 		void *au, const void *gf, const void *mass, const void *dmat,
 		double lambda, const int *bc, int apply_mask, const int *done,
 		double *part, const PUpd *pu)
 {
-	// the deferred solution step (PU = 2) is instantiated for FP64 fields
-	// only, where the fused CG takes it
-	if (pu && pu->u && sizeof(T) == 8)
-		launch_ax1<N, T, G, (sizeof(T) == 8 ? 2 : 1), V>(st, nel, op, u, au,
-				gf, mass, dmat, lambda, bc, apply_mask, done, part, *pu);
-	else if (pu)
-		launch_ax1<N, T, G, 1, V>(st, nel, op, u, au, gf, mass, dmat,
-				lambda, bc, apply_mask, done, part, *pu);
-	else
-		launch_ax1<N, T, G, 0, V>(st, nel, op, u, au, gf, mass, dmat,
-				lambda, bc, apply_mask, done, part, PUpd{ nullptr, nullptr,
-				nullptr, 0, -1, nullptr, 0, ssx_replay{} });
+	// FP64 from 9 to 12 points: one element a workgroup on the matrix
+	// instruction where that is faster (ssx_axm.h); of the shape only the
+	// streaming hint is left
+	if constexpr (axm_takes<N, T>) {
+		if (axm_use<N>(nel)) {
+			constexpr bool NT = (V & 2) != 0;
+			if (pu && pu->u)
+				launch_axm<N, 2, NT>(st, nel, op, u, au, gf, mass, dmat,
+						lambda, bc, apply_mask, done, part, *pu);
+			else if (pu)
+				launch_axm<N, 1, NT>(st, nel, op, u, au, gf, mass, dmat,
+						lambda, bc, apply_mask, done, part, *pu);
+			else
+				launch_axm<N, 0, NT>(st, nel, op, u, au, gf, mass, dmat,
+						lambda, bc, apply_mask, done, part, PUpd{ nullptr,
+						nullptr, nullptr, 0, -1, nullptr, 0, ssx_replay{} });
+			return;
+		}
+	}
+	if constexpr (!(axm_takes<N, T> && N == 12)) {
+		// the deferred solution step (PU = 2) is instantiated for FP64
+		// fields only, where the fused CG takes it
+		if (pu && pu->u && sizeof(T) == 8)
+			launch_ax1<N, T, G, (sizeof(T) == 8 ? 2 : 1), V>(st, nel, op, u,
+					au, gf, mass, dmat, lambda, bc, apply_mask, done, part,
+					*pu);
+		else if (pu)
+			launch_ax1<N, T, G, 1, V>(st, nel, op, u, au, gf, mass, dmat,
+					lambda, bc, apply_mask, done, part, *pu);
+		else
+			launch_ax1<N, T, G, 0, V>(st, nel, op, u, au, gf, mass, dmat,
+					lambda, bc, apply_mask, done, part, PUpd{ nullptr,
+					nullptr, nullptr, 0, -1, nullptr, 0, ssx_replay{} });
+	}
 }
 
 // dispatcher body shared by the per-precision files: n in [2,16], variant

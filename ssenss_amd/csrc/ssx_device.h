@@ -54,6 +54,15 @@ __device__ __forceinline__ T *gptr(T *p)
 	return (T *) (SSX_GLOBAL T *) (unsigned long long) p;
 }
 
+// the same value, hidden from the compiler: it would otherwise compute the
+// addresses of every phase (or loop turn) from the lane number once, keep
+// them in registers throughout and spill
+__device__ __forceinline__ int fresh(int x)
+{
+	asm volatile("" : "+v"(x));
+	return x;
+}
+
 // Logical workgroup of a gather kernel.  Workgroups go to the 8 XCDs
 // round-robin (workgroup b on XCD b % 8), and each XCD has its own L2.
 // Renumbering so that XCD x takes a contiguous range of logical workgroups

@@ -205,15 +205,6 @@ struct ConvShape {
 // l / 16
 #define CONV_ROW(r) (4 * (r) + kq)
 
-// the same value, hidden from the compiler: it would otherwise compute the
-// addresses of every phase from the lane number once, keep them in
-// registers throughout and spill (97 registers at N = 10)
-__device__ __forceinline__ int fresh(int x)
-{
-	asm volatile("" : "+v"(x));
-	return x;
-}
-
 // one contraction of three components: for every line l < C of component f,
 // dst(f, l)[m * SM] = sum_k a[m][k] src(f, l)[k], m < M, k < K.  A
 // wavefront takes its tiles of 16 lines together (all loads, then the
