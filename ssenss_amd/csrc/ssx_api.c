@@ -1773,15 +1773,10 @@ int ssx_fcg_iter(ssx_ctx *c, int op, int var, double *u, ssx_fcg_state *s)
 		ap[k] = ap[k - 1];
 	ap[0] = ta;
 	TRY(ssx_opeval(c, 0, op, var, p[0], ap[0]));
-	for (int k = m2 - 1; k > 0; --k)
-		TRY(ssxk_scalar(st, c->scal, 2, SC_PAP0 + k, SC_PAP0 + k - 1, 0,
-				0.0));
-	/* <p_0, Ap_0>_w and <p_0, r>_w in one pass */
-	const double *pr2[2] = { ap[0], r };
-	TRY(ssxk_multidot(st, nt, p[0], L->scale, pr2, 2, c->part, c->scal,
-			SC_PAPN, -1, 0));
-	TRY(ssxk_scalar(st, c->scal, 2, SC_PAP0, SC_PAPN, 0, 0.0));
-	TRY(ssxk_scalar(st, c->scal, 0, SC_ALPHA, SC_PAPN + 1, SC_PAPN, 0.0));
+	/* <p_0, Ap_0>_w and <p_0, r>_w in one pass, alpha, and the history's
+	 * <p_k, Ap_k> moved up */
+	TRY(ssxk_fcg_pair(st, nt, p[0], L->scale, ap[0], r, c->part, c->scal,
+			m2 - 1));
 	/* u += alpha p_0; r -= alpha Ap_0; <r,r>_w */
 	TRY(ssxk_fcg_step(st, nt, c->scal, SC_ALPHA, p[0], ap[0], u, r,
 			L->scale, c->part));

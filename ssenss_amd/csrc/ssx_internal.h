@@ -455,12 +455,16 @@ int ssxk_cg_reduce1(void *stream, const double *part, long long cnt,
 int ssxk_cg_tol(void *stream, double *scal, int dst, int src, double eps,
 		double rtol);
 int ssxk_set_ints(void *stream, int *dst, int v, int n);
-/* FCG: scal[dst+k] = <x, ys[k]>_w for k < m (each bit-identical to
- * ssxk_dot + ssxk_reduce); div >= 0: scal[quot+k] = scal[dst+k] /
- * scal[div+k] */
+/* FCG: scal[dst+k] = <x, ys[k]>_w for k < m (the same bits
+ * for every m) and scal[quot+k] = scal[dst+k] / scal[div+k] */
 int ssxk_multidot(void *stream, size_t n, const double *x, const double *s,
 		const double *const *ys, int m, double *part, double *scal, int dst,
 		int div, int quot);
+/* FCG: <p,ap>_w and <p,r>_w into SC_PAPN, SC_PAPN+1, their quotient into
+ * SC_ALPHA, SC_PAP0..+shift-1 moved up by one and <p,ap>_w put first */
+int ssxk_fcg_pair(void *stream, size_t n, const double *p, const double *s,
+		const double *ap, const double *r, double *part, double *scal,
+		int shift);
 /* y = mask * (x - sum_k scal[ib+k] ps[k]), k = 0..m-1 in order */
 int ssxk_multi_axpy(void *stream, size_t n, const double *x,
 		const double *const *ps, int m, const double *scal, int ib,

@@ -1512,41 +1512,80 @@ extern "C" int ssxk_reduce(void *stream, double *part, int slot, double *scal,
 // ---------------------------------------------------------------------
 // Flexible CG (solver.c:83-157) orthogonalisation, fused: each kernel
 // reads every vector once.  Per-thread accumulation order, grid and tree
-// are those of k_dot / k_reduce, so every inner product is bit-identical
-// to the one-dot-per-launch sequence.
+// are those of k_dot / k_reduce (a term enters by one fused multiply-add
+// here, by a product and a sum there), whatever the number of vectors.
 // ---------------------------------------------------------------------
 
 struct VecSet {
 	const double *v[SSX_FCG_M];
 };
 
-// part[k*NPART + blk] = block partial of <x, y_k>_w, k < m
+// part[k*NPART + blk] = block partial of <x, y_k>_w, k < M.
+// Bound by the M + 2 vectors it reads once.  M is a template argument: with
+// the count at run time each vector's load stood behind a test of its own
+// and was waited for before the next went out (one load in flight a
+// wavefront): 16.8 million nodes took 156 us at M = 3 and 398 at M = 10, 4.3
+// and 4.1 TB/s.  Here the loads of U rows of nodes go out together, U so that
+// about 24 are in flight: 112 and 266 us, 6.0 TB/s; 2.3 million nodes at M =
+// 10 47.5 -> 36.2 us.  Each sum still takes its terms in k_dot's order.  The
+// M trees run side by side, one barrier a level for all (32768 nodes, M = 10:
+// 13.1 -> 8.3 us with the reduction).
+template <int M>
 __global__ void __launch_bounds__(256)
 k_multidot(size_t n, const double *__restrict__ x,
-		const double *__restrict__ s, VecSet ys, int m,
-		double *__restrict__ part)
+		const double *__restrict__ s, VecSet ys, double *__restrict__ part)
 {
-	__shared__ double sh[256];
-	double acc[SSX_FCG_M];
+	constexpr int U = M <= 2 ? 6 : M <= 4 ? 4 : M <= 8 ? 3 : 2;
+	__shared__ double sh[M][256];
+	const size_t stride = (size_t) gridDim.x * 256;
+	const int t = threadIdx.x;
+	double acc[M];
 #pragma unroll
-	for (int k = 0; k < SSX_FCG_M; ++k)
+	for (int k = 0; k < M; ++k)
 		acc[k] = 0.0;
-	GRID_STRIDE(q, n) {
+	size_t q = (size_t) blockIdx.x * 256 + t;
+	for (; q + (U - 1) * stride < n; q += U * stride) {
+		double xv[U], sv[U], yv[U][M];
+#pragma unroll
+		for (int i = 0; i < U; ++i) {
+			xv[i] = x[q + i * stride];
+			sv[i] = s[q + i * stride];
+#pragma unroll
+			for (int k = 0; k < M; ++k)
+				yv[i][k] = ys.v[k][q + i * stride];
+		}
+#pragma unroll
+		for (int i = 0; i < U; ++i) {
+			const double a = xv[i] * sv[i];
+#pragma unroll
+			for (int k = 0; k < M; ++k)
+				acc[k] += a * yv[i][k];
+		}
+	}
+	for (; q < n; q += stride) {
 		const double a = x[q] * s[q];
 #pragma unroll
-		for (int k = 0; k < SSX_FCG_M; ++k)
-			if (k < m)
-				acc[k] += a * ys.v[k][q];
+		for (int k = 0; k < M; ++k)
+			acc[k] += a * ys.v[k][q];
 	}
-	for (int k = 0; k < m; ++k) {
-		const double t = block_sum256(acc[k], sh);
-		if (threadIdx.x == 0)
-			part[(size_t) k * SSX_NPART + blockIdx.x] = t;
+	// block_sum256's tree for each sum
+#pragma unroll
+	for (int k = 0; k < M; ++k)
+		sh[k][t] = acc[k];
+	__syncthreads();
+	for (int st = 128; st > 0; st >>= 1) {
+		if (t < st) {
+#pragma unroll
+			for (int k = 0; k < M; ++k)
+				sh[k][t] += sh[k][t + st];
+		}
 		__syncthreads();
 	}
+	if (t < M)
+		part[(size_t) t * SSX_NPART + blockIdx.x] = sh[t][0];
 }
 
-// block k: scal[dst + k] = sum of part[k*NPART ..]; with div >= 0 also
+// block k: scal[dst + k] = sum of part[k*NPART ..] and
 // scal[quot + k] = scal[dst + k] / scal[div + k]
 __global__ void __launch_bounds__(256)
 k_reduce_multi(const double *__restrict__ part, double *__restrict__ scal,
@@ -1560,8 +1599,38 @@ k_reduce_multi(const double *__restrict__ part, double *__restrict__ scal,
 	const double t = block_sum256(acc, sh);
 	if (threadIdx.x == 0) {
 		scal[dst + blockIdx.x] = t;
-		if (div >= 0)
-			scal[quot + blockIdx.x] = t / scal[div + blockIdx.x];
+		scal[quot + blockIdx.x] = t / scal[div + blockIdx.x];
+	}
+}
+
+// One block, after the pair <p,Ap>_w, <p,r>_w of k_multidot<2>: both sums
+// (k_reduce_multi's), the history's <p_k,Ap_k> moved up by one (shift of
+// them), the new one put first, and alpha = <p,r> / <p,Ap>.  Each of these
+// had a launch of its own, up to 12 an iteration, 2.3 to 4.6 us each.
+__global__ void __launch_bounds__(256)
+k_fcg_scalars(const double *__restrict__ part, double *__restrict__ scal,
+		int shift)
+{
+	__shared__ double sh[256];
+	const int t = threadIdx.x;
+	const double old = t < shift ? scal[SC_PAP0 + t] : 0.0;
+	double sum[2];
+	for (int k = 0; k < 2; ++k) {
+		const double *pp = part + (size_t) k * SSX_NPART;
+		double acc = 0.0;
+#pragma unroll
+		for (int q = 0; q < SSX_NPART / 256; ++q)
+			acc += pp[t + q * 256];
+		sum[k] = block_sum256(acc, sh);
+		__syncthreads();
+	}
+	if (t < shift)
+		scal[SC_PAP0 + t + 1] = old;
+	if (t == 0) {
+		scal[SC_PAPN] = sum[0];
+		scal[SC_PAPN + 1] = sum[1];
+		scal[SC_PAP0] = sum[0];
+		scal[SC_ALPHA] = sum[1] / sum[0];
 	}
 }
 
@@ -1599,12 +1668,37 @@ extern "C" int ssxk_multidot(void *stream, size_t n, const double *x,
 	VecSet v;
 	for (int k = 0; k < SSX_FCG_M; ++k)
 		v.v[k] = k < m ? ys[k] : ys[0];
-	hipLaunchKernelGGL(k_multidot, dim3(SSX_NPART), dim3(256), 0,
-			(hipStream_t) stream, n, x, s, v, m, part);
+#define MDOT(M)                                                              \
+	case M:                                                              \
+		hipLaunchKernelGGL(k_multidot<M>, dim3(SSX_NPART), dim3(256),    \
+				0, (hipStream_t) stream, n, x, s, v, part);  \
+		break;
+	switch (m) {
+	MDOT(1) MDOT(2) MDOT(3) MDOT(4) MDOT(5)
+	MDOT(6) MDOT(7) MDOT(8) MDOT(9) MDOT(10)
+	}
+	static_assert(SSX_FCG_M == 10, "every length of the history");
+#undef MDOT
 	LAUNCH_CHECK("k_multidot");
 	hipLaunchKernelGGL(k_reduce_multi, dim3(m), dim3(256), 0,
 			(hipStream_t) stream, part, scal, dst, div, quot);
 	LAUNCH_CHECK("k_reduce_multi");
+	return SSX_OK;
+}
+
+extern "C" int ssxk_fcg_pair(void *stream, size_t n, const double *p,
+		const double *s, const double *ap, const double *r, double *part,
+		double *scal, int shift)
+{
+	VecSet v;
+	for (int k = 0; k < SSX_FCG_M; ++k)
+		v.v[k] = k == 0 ? ap : r;
+	hipLaunchKernelGGL(k_multidot<2>, dim3(SSX_NPART), dim3(256), 0,
+			(hipStream_t) stream, n, p, s, v, part);
+	LAUNCH_CHECK("k_multidot");
+	hipLaunchKernelGGL(k_fcg_scalars, dim3(1), dim3(256), 0,
+			(hipStream_t) stream, part, scal, shift);
+	LAUNCH_CHECK("k_fcg_scalars");
 	return SSX_OK;
 }
 
