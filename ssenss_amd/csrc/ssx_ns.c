@@ -69,6 +69,15 @@ int ssxk_ns_comb(void *st, size_t nt, const double *const x[3][3],
 		const double a[3], const int use[3], double *const y[3]);
 int ssxk_ns_mul3(void *st, size_t nt, double alpha, const double *const x[3],
 		const double *const w[3], double beta, double *const z[3]);
+int ssxk_ns_rk_stage(void *st, size_t nt, int ncomp, int nterm,
+		const double *const x[3][3], const double co[3],
+		const double *const ut[3], const double *const f[3],
+		const double *im, double ch, double *const a[3],
+		double *const y[3]);
+int ssxk_ns_rk_end(void *st, size_t nt, double *const f[4][3],
+		const double *im, double c0, double c1, double *const ut[3]);
+int ssxk_ns_dss3(void *st, int *const grp[3], const long long ng[3],
+		double *const u[3]);
 
 struct ssx_ns {
 	ssx_ctx *c;
@@ -85,7 +94,7 @@ struct ssx_ns {
 	double *u[3][3], *p[3], *conv[3][3], *rot[3][3];
 	/* scratch at n */
 	double *ut[3], *rhs[3], *a[3], *b[3], *J[9];
-	double *rkf[4][3], *rky[4][3];
+	double *rkf[4][3], *rky[3];
 	int inited;
 	long long cnt_solve[4];
 };
@@ -114,7 +123,7 @@ void ssx_ns_destroy(ssx_ns *ns)
 	if (ns->vb)
 		ssx_batch_destroy(ns->vb);
 	double **all[] = { ns->ti, ns->ti + 3, ns->ti + 6, ns->wn, ns->ut,
-		ns->rhs, ns->a, ns->b, ns->J, ns->J + 3, ns->J + 6, ns->p };
+		ns->rhs, ns->a, ns->b, ns->rky, ns->J, ns->J + 3, ns->J + 6, ns->p };
 	for (size_t k = 0; k < sizeof(all) / sizeof(all[0]); ++k)
 		for (int c = 0; c < 3; ++c)
 			hipFree(all[k][c]);
@@ -127,7 +136,6 @@ void ssx_ns_destroy(ssx_ns *ns)
 	for (int s = 0; s < 4; ++s)
 		for (int c = 0; c < 3; ++c) {
 			hipFree(ns->rkf[s][c]);
-			hipFree(ns->rky[s][c]);
 		}
 	hipFree(ns->dm_c);
 	hipFree(ns->prol_c);
@@ -354,11 +362,10 @@ int ssx_ns_create(ssx_ns **out, ssx_ctx *c, const ssx_ns_params *prm)
 			&ns->b[d] };
 		for (int k = 0; k < 5 && rc == SSX_OK; ++k)
 			rc = nalloc(v[k], nt);
-		for (int s = 0; s < 4 && rc == SSX_OK; ++s) {
+		if (rc == SSX_OK)
+			rc = nalloc(&ns->rky[d], nt);
+		for (int s = 0; s < 4 && rc == SSX_OK; ++s)
 			rc = nalloc(&ns->rkf[s][d], nt);
-			if (rc == SSX_OK)
-				rc = nalloc(&ns->rky[s][d], nt);
-		}
 	}
 	for (int k = 0; k < 9 && rc == SSX_OK; ++k)
 		rc = nalloc(&ns->J[k], nt);
@@ -426,26 +433,36 @@ static int ns_double_curl(ssx_ns *ns, double *const u[3], double *const out[3])
 			out);
 }
 
-/* y += alpha U(t), the velocity history interpolated to time t with
- * Lagrange weights, terms of weight |w| <= 1e-6 left out
- * (add_interpolated_velocity, time.c:132-152) */
-static int ns_add_interp(ssx_ns *ns, double *const y[3], double t,
-		double alpha)
+/* U(t), the velocity history interpolated to time t with Lagrange weights,
+ * terms of weight |w| <= 1e-6 left out (add_interpolated_velocity,
+ * time.c:132-152): the terms' fields and alpha times their weights; returns
+ * their number */
+static int ns_interp(const ssx_ns *ns, double t, double alpha,
+		const double *x[3][3], double co[3])
 {
 	const double t0 = ns->t, dt0 = ns->dt;
 	const double d[3] = { t - t0 + 2.0 * dt0, t - t0 + dt0, t - t0 };
-	const double a = 0.5 * d[1] * d[2] / pow(dt0, 2);
-	const double b = -d[0] * d[2] / pow(dt0, 2);
-	const double c = 0.5 * d[0] * d[1] / pow(dt0, 2);
-	const double eps = 1.0e-6;
-	const double *x[3][3];
-	for (int k = 0; k < 3; ++k) {
-		x[0][k] = ns->u[2][k];
-		x[1][k] = ns->u[1][k];
-		x[2][k] = ns->u[0][k];
+	const double w[3] = { 0.5 * d[1] * d[2] / pow(dt0, 2),
+		-d[0] * d[2] / pow(dt0, 2), 0.5 * d[0] * d[1] / pow(dt0, 2) };
+	int m = 0;
+	for (int l = 0; l < 3; ++l) {
+		if (!(fabs(w[l]) > 1.0e-6))
+			continue;
+		for (int k = 0; k < 3; ++k)
+			x[m][k] = ns->u[2 - l][k];
+		co[m++] = w[l] * alpha;
 	}
-	const double co[3] = { a * alpha, b * alpha, c * alpha };
-	const int use[3] = { fabs(a) > eps, fabs(b) > eps, fabs(c) > eps };
+	return m;
+}
+
+/* y += alpha U(t) */
+static int ns_add_interp(ssx_ns *ns, double *const y[3], double t,
+		double alpha)
+{
+	const double *x[3][3] = { { NULL } };
+	double co[3] = { 0.0, 0.0, 0.0 };
+	const int m = ns_interp(ns, t, alpha, x, co);
+	const int use[3] = { m > 0, m > 1, m > 2 };
 	return ssxk_ns_comb(ns->c->stream, ns->nt, x, co, use, y);
 }
 
@@ -456,47 +473,42 @@ static int ns_inv_mass(ssx_ns *ns, double *const f[3])
 	ssx_ctx *c = ns->c;
 	const ssx_level *L = &c->lev[0];
 	const double *im[3] = { c->inv_mass, c->inv_mass, c->inv_mass };
-	for (int d = 0; d < 3; ++d)
-		TRYN(ssxk_dss_all(c->stream, L->grp, L->ngrp, f[d], NULL, NULL, 0,
-				NULL));
+	TRYN(ssxk_ns_dss3(c->stream, L->grp, L->ngrp, f));
 	return ssxk_ns_mul3(c->stream, ns->nt, 1.0, (const double *const *) f,
 			im, 0.0, f);
 }
 
-/* integrate_convection_rk4 (time.c:84-130) on ut */
+/* integrate_convection_rk4 (time.c:84-130) on ut.  The inverse mass of a
+ * stage's operator is applied where the stage is read.  The velocity of a
+ * stage (in a) serves every stage in a row at the same time. */
 static int ns_rk4(ssx_ns *ns, double t0, double t, double h, double beta)
 {
 	void *st = ns->c->stream;
+	const ssx_level *L = &ns->c->lev[0];
 	static const double ra[4] = { 0.0, 0.5, 0.5, 1.0 };
-	static const double rb[4] = { 1.0, 2.0, 2.0, 1.0 };
+	const double *im = ns->c->inv_mass;
+	const double *const *ut = (const double *const *) ns->ut;
 	const size_t nt = ns->nt;
 	TRYN(ns_add_interp(ns, ns->ut, t0, beta));
+	double ta = NAN;
 	int k = 0;
 	while (t0 + (double) k++ * h < t - 0.5 * h) {
 		for (int i = 0; i < 4; ++i) {
-			for (int d = 0; d < 3; ++d)
-				TRYN(ssxk_copy(st, ns->rky[i][d], ns->ut[d], nt));
-			if (i > 0) {
-				const double *x[3][3] = { { ns->rkf[i - 1][0],
-					ns->rkf[i - 1][1], ns->rkf[i - 1][2] } };
-				const double co[3] = { -h * ra[i], 0.0, 0.0 };
-				const int use[3] = { 1, 0, 0 };
-				TRYN(ssxk_ns_comb(st, nt, x, co, use, ns->rky[i]));
-			}
-			for (int d = 0; d < 3; ++d)
-				TRYN(ssxk_fill(st, ns->a[d], 0.0, nt));
-			TRYN(ns_add_interp(ns, ns->a, t0 + ((double) (k - 1) + ra[i])
-					* h, 1.0));
-			TRYN(ns_convection(ns, ns->a, ns->rky[i], ns->rkf[i]));
-			TRYN(ns_inv_mass(ns, ns->rkf[i]));
+			const double ts = t0 + ((double) (k - 1) + ra[i]) * h;
+			const double *x[3][3] = { { NULL } };
+			double co[3] = { 0.0, 0.0, 0.0 };
+			const int m = ts == ta ? 0 : ns_interp(ns, ts, 1.0, x, co);
+			if (m > 0 || i > 0)
+				TRYN(ssxk_ns_rk_stage(st, nt, 3, m, x, co, ut, i == 0 ? NULL
+						: (const double *const *) ns->rkf[i - 1], im,
+						-h * ra[i], ns->a, ns->rky));
+			ta = ts;
+			TRYN(ns_convection(ns, ns->a, i == 0 ? ns->ut : ns->rky,
+					ns->rkf[i]));
+			TRYN(ssxk_ns_dss3(st, L->grp, L->ngrp, ns->rkf[i]));
 		}
-		for (int i = 0; i < 4; ++i) {
-			const double *x[3][3] = { { ns->rkf[i][0], ns->rkf[i][1],
-				ns->rkf[i][2] } };
-			const double co[3] = { -h * rb[i] / 6.0, 0.0, 0.0 };
-			const int use[3] = { 1, 0, 0 };
-			TRYN(ssxk_ns_comb(st, nt, x, co, use, ns->ut));
-		}
+		TRYN(ssxk_ns_rk_end(st, nt, ns->rkf, im, -h * 1.0 / 6.0,
+				-h * 2.0 / 6.0, ns->ut));
 	}
 	return SSX_OK;
 }
@@ -606,21 +618,16 @@ int ssx_ns_step(ssx_ns *ns, ssx_stats stats[4])
 	}
 	/* estimate_pressure (navier_stokes.c:101-113) and the solve */
 	{
-		/* the three-component combination on (p, p, p): the three
-		 * outputs are equal, a[0] is kept */
-		const double *x[3][3] = { { ns->p[0], ns->p[0], ns->p[0] },
-			{ ns->p[1], ns->p[1], ns->p[1] },
-			{ ns->p[2], ns->p[2], ns->p[2] } };
-		for (int d = 0; d < 3; ++d)
-			TRYN(ssxk_fill(st, ns->a[d], 0.0, nt));
+		/* into the oldest level, which becomes the newest */
+		const double *x[3][3] = { { ns->p[0] }, { ns->p[1] },
+			{ ns->p[2] } };
 		const double co[3] = { 3.0, -3.0, 1.0 };
-		const int use[3] = { 1, 1, 1 };
-		TRYN(ssxk_ns_comb(st, nt, x, co, use, ns->a));
+		TRYN(ssxk_ns_rk_stage(st, nt, 1, 3, x, co, NULL, NULL, NULL, 0.0,
+				ns->p + 2, NULL));
 		double *tp = ns->p[2];
 		ns->p[2] = ns->p[1];
 		ns->p[1] = ns->p[0];
 		ns->p[0] = tp;
-		TRYN(ssxk_copy(st, ns->p[0], ns->a[0], nt));
 	}
 	int rc = ssx_fcg(c, SSX_OP_POISSON, SSX_PRESSURE, SSX_PC_MG, ns->rhs[0],
 			ns->p[0], NS_TOL, 5000, &sloc[0]);
@@ -645,23 +652,18 @@ int ssx_ns_step(ssx_ns *ns, ssx_stats stats[4])
 		const int use[3] = { 1, 0, 0 };
 		TRYN(ssxk_ns_comb(st, nt, x, co, use, ns->rhs));
 	}
-	for (int d = 0; d < 3; ++d)
-		TRYN(ssxk_dss_all(st, L->grp, L->ngrp, ns->rhs[d], NULL, NULL, 0,
-				NULL));
+	TRYN(ssxk_ns_dss3(st, L->grp, L->ngrp, ns->rhs));
 	/* estimate_velocity (navier_stokes.c:161-175) */
 	{
+		/* into the oldest level, which becomes the newest */
 		const double *x[3][3];
 		for (int l = 0; l < 3; ++l)
 			for (int d = 0; d < 3; ++d)
 				x[l][d] = ns->u[l][d];
-		for (int d = 0; d < 3; ++d)
-			TRYN(ssxk_fill(st, ns->a[d], 0.0, nt));
 		const double co[3] = { 3.0, -3.0, 1.0 };
-		const int use[3] = { 1, 1, 1 };
-		TRYN(ssxk_ns_comb(st, nt, x, co, use, ns->a));
+		TRYN(ssxk_ns_rk_stage(st, nt, 3, 3, x, co, NULL, NULL, NULL, 0.0,
+				ns->u[2], NULL));
 		rotate3(ns->u);
-		for (int d = 0; d < 3; ++d)
-			TRYN(ssxk_copy(st, ns->u[0][d], ns->a[d], nt));
 		TRYN(ssxk_ns_zero_dir(st, nt, ns->n, L->bc, ns->u[0]));
 	}
 	/* the three Helmholtz solves (navier_stokes.c:218-221) */

@@ -613,6 +613,191 @@ k_ns_mul3(long long nt, double alpha, P3 x, P3 w, double beta, M3 z)
 	}
 }
 
+// One stage of the convection RK4 (time.c:84-130), per node and component
+// (blockIdx.y): a = sum of T terms co_t x_t, the velocity at the stage's time
+// (from zero, in order), and with STAGE y = ut + ch (im f), the stage's
+// argument, im f being the inverse mass applied to the last stage's f.
+// With T alone it is any such sum; a may be one of the x.
+// Bound by the T + 1 (+ 4) values it moves (T = 3 with STAGE: 311 us on 9.2
+// million nodes, 5.7 TB/s).  The stage had 13 launches: three copies, three
+// fills, two sums read and written in place, one DSS a component, the
+// inverse mass; 2 to 5 us each on 512 elements of 8 points, 0.83 ms
+// together on the 9.2 million nodes.  Now this, the operator and one DSS,
+// and a velocity formed once for the stages at one time: 0.43 ms.
+struct RkTerms {
+	const double *x[3][3];    // [term][component]
+	double co[3];
+};
+
+template <int T, bool STAGE>
+__global__ void __launch_bounds__(256)
+k_ns_rk_stage(long long nt, RkTerms rk, P3 ut, P3 f,
+		const double *__restrict__ im, double ch, M3 a, M3 y)
+{
+	const long long q = (long long) blockIdx.x * 256 + threadIdx.x;
+	const int c = blockIdx.y;
+	if (q >= nt)
+		return;
+	double xv[T > 0 ? T : 1], uv = 0.0, fv = 0.0, mv = 0.0;
+#pragma unroll
+	for (int t = 0; t < T; ++t)
+		xv[t] = rk.x[t][c][q];
+	if (STAGE) {
+		uv = ut.p[c][q];
+		fv = f.p[c][q];
+		mv = im[q];
+	}
+	if (T > 0) {
+		double v = 0.0;
+#pragma unroll
+		for (int t = 0; t < T; ++t)
+			v = rk.co[t] * xv[t] + v;
+		a.p[c][q] = v;
+	}
+	if (STAGE) {
+		const double g = __dmul_rn(fv, mv);
+		y.p[c][q] = ch * g + uv;
+	}
+}
+
+// ut += sum of the four stages, in order, the inverse mass applied to each
+__global__ void __launch_bounds__(256)
+k_ns_rk_end(long long nt, P3 f0, P3 f1, P3 f2, P3 f3,
+		const double *__restrict__ im, double c0, double c1, M3 ut)
+{
+	const long long q = (long long) blockIdx.x * 256 + threadIdx.x;
+	const int c = blockIdx.y;
+	if (q >= nt)
+		return;
+	const double mv = im[q];
+	const double g0 = __dmul_rn(f0.p[c][q], mv);
+	const double g1 = __dmul_rn(f1.p[c][q], mv);
+	const double g2 = __dmul_rn(f2.p[c][q], mv);
+	const double g3 = __dmul_rn(f3.p[c][q], mv);
+	double v = ut.p[c][q];
+	v = c0 * g0 + v;
+	v = c1 * g1 + v;
+	v = c1 * g2 + v;
+	ut.p[c][q] = c0 * g3 + v;
+}
+
+// dss_group on three fields: the group's list read once, the three sums of
+// a copy in dss_group's order
+template <int M>
+__device__ __forceinline__ void dss3_group(long long G, long long g,
+		const int *__restrict__ idx, M3 u)
+{
+	int ix[M];
+	double v[3][M];
+#pragma unroll
+	for (int t = 0; t < M; ++t)
+		ix[t] = idx[(long long) t * G + g];
+#pragma unroll
+	for (int c = 0; c < 3; ++c)
+#pragma unroll
+		for (int t = 0; t < M; ++t)
+			v[c][t] = u.p[c][ix[t]];
+#pragma unroll
+	for (int c = 0; c < 3; ++c)
+#pragma unroll
+		for (int t = 0; t < M; ++t) {
+			double s = v[c][t];
+#pragma unroll
+			for (int k = 1; k < M; ++k)
+				s = s + v[c][t ^ dss_ord(M, k)];
+			u.p[c][ix[t]] = s;
+		}
+}
+
+// k_dss_all on three fields in one launch
+__global__ void __launch_bounds__(256)
+k_ns_dss3(long long G2, long long G4, long long G8,
+		const int *__restrict__ i2, const int *__restrict__ i4,
+		const int *__restrict__ i8, M3 u)
+{
+	const long long b2 = (G2 + 255) / 256, b4 = (G4 + 255) / 256;
+	const long long b = blockIdx.x;
+	if (b < b2) {
+		const long long g = b * 256 + threadIdx.x;
+		if (g < G2)
+			dss3_group<2>(G2, g, i2, u);
+	} else if (b < b2 + b4) {
+		const long long g = (b - b2) * 256 + threadIdx.x;
+		if (g < G4)
+			dss3_group<4>(G4, g, i4, u);
+	} else {
+		const long long g = (b - b2 - b4) * 256 + threadIdx.x;
+		if (g < G8)
+			dss3_group<8>(G8, g, i8, u);
+	}
+}
+
+// nterm 0..3 terms; f NULL: no stage argument; ncomp components
+extern "C" int ssxk_ns_rk_stage(void *st, size_t nt, int ncomp, int nterm,
+		const double *const x[3][3], const double co[3],
+		const double *const ut[3], const double *const f[3],
+		const double *im, double ch, double *const a[3], double *const y[3])
+{
+	RkTerms rk;
+	P3 pu, pf;
+	M3 pa, py;
+	for (int c = 0; c < 3; ++c) {
+		for (int t = 0; t < 3; ++t)
+			rk.x[t][c] = t < nterm && c < ncomp ? x[t][c] : nullptr;
+		pu.p[c] = f ? ut[c] : nullptr;
+		pf.p[c] = f ? f[c] : nullptr;
+		pa.p[c] = nterm && c < ncomp ? a[c] : nullptr;
+		py.p[c] = f ? y[c] : nullptr;
+		rk.co[c] = c < nterm ? co[c] : 0.0;
+	}
+	const dim3 grid(ns_blocks(nt), (unsigned) ncomp);
+#define RKCASE(T, F)                                                         \
+	case 2 * T + F:                                                      \
+		hipLaunchKernelGGL((k_ns_rk_stage<T, F>), grid, dim3(256), 0,    \
+				(hipStream_t) st, (long long) nt, rk, pu, pf, im, ch, \
+				pa, py);                                     \
+		break;
+	switch (2 * nterm + (f ? 1 : 0)) {
+	RKCASE(0, 1) RKCASE(1, 0) RKCASE(1, 1) RKCASE(2, 0) RKCASE(2, 1)
+	RKCASE(3, 0) RKCASE(3, 1)
+	default:
+		break;                          // nothing asked for
+	}
+#undef RKCASE
+	NS_LAUNCH("k_ns_rk_stage");
+	return SSX_OK;
+}
+
+extern "C" int ssxk_ns_rk_end(void *st, size_t nt,
+		double *const f[4][3], const double *im, double c0, double c1,
+		double *const ut[3])
+{
+	P3 pf[4];
+	for (int i = 0; i < 4; ++i)
+		for (int c = 0; c < 3; ++c)
+			pf[i].p[c] = f[i][c];
+	M3 pu = { { ut[0], ut[1], ut[2] } };
+	hipLaunchKernelGGL(k_ns_rk_end, dim3(ns_blocks(nt), 3), dim3(256), 0,
+			(hipStream_t) st, (long long) nt, pf[0], pf[1], pf[2], pf[3], im,
+			c0, c1, pu);
+	NS_LAUNCH("k_ns_rk_end");
+	return SSX_OK;
+}
+
+extern "C" int ssxk_ns_dss3(void *st, int *const grp[3],
+		const long long ng[3], double *const u[3])
+{
+	const long long nb = ssxk_dss_blocks(ng);
+	M3 pu = { { u[0], u[1], u[2] } };
+	if (nb == 0)
+		return SSX_OK;
+	hipLaunchKernelGGL(k_ns_dss3, dim3((unsigned) nb), dim3(256), 0,
+			(hipStream_t) st, ng[0], ng[1], ng[2], grp[0], grp[1], grp[2],
+			pu);
+	NS_LAUNCH("k_ns_dss3");
+	return SSX_OK;
+}
+
 extern "C" int ssxk_ns_jac(void *st, size_t nt, int n, const double *dm,
 		const double *const a[3], double *const out[9])
 {
