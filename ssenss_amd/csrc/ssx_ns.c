@@ -48,14 +48,13 @@
 #define NS_TOL 1.0e-10          /* residual_tolerance, navier_stokes.c:33-99 */
 
 /* kernels (ssx_nskernels.hip) */
-int ssxk_ns_jac(void *st, size_t nt, int n, const double *dm,
-		const double *const a[3], double *const out[9]);
-int ssxk_ns_curl(void *st, size_t nt, const double *const J[9],
-		const double *const ti[9], const double *mass, double *const out[3]);
-int ssxk_ns_div(void *st, size_t nt, const double *const J[9],
-		const double *const ti[9], const double *mass, double scale,
-		double *out);
-int ssxk_ns_grad(void *st, size_t nt, int n, const double *dm,
+int ssxk_ns_curl(void *st, int nel, int n, const double *dm,
+		const double *const a[3], const double *const ti[9],
+		const double *mass, double *const out[3]);
+int ssxk_ns_div(void *st, int nel, int n, const double *dm,
+		const double *const a[3], const double *const ti[9],
+		const double *mass, double scale, double *out);
+int ssxk_ns_grad(void *st, int nel, int n, const double *dm,
 		const double *p, const double *mass, const double *const ti[9],
 		double *const out[3]);
 int ssxk_ns_conv(void *st, int nel, int n, const double *prol,
@@ -93,7 +92,7 @@ struct ssx_ns {
 	/* fields: [0] newest level */
 	double *u[3][3], *p[3], *conv[3][3], *rot[3][3];
 	/* scratch at n */
-	double *ut[3], *rhs[3], *a[3], *b[3], *J[9];
+	double *ut[3], *rhs[3], *a[3], *b[3];
 	double *rkf[4][3], *rky[3];
 	int inited;
 	long long cnt_solve[4];
@@ -123,7 +122,7 @@ void ssx_ns_destroy(ssx_ns *ns)
 	if (ns->vb)
 		ssx_batch_destroy(ns->vb);
 	double **all[] = { ns->ti, ns->ti + 3, ns->ti + 6, ns->wn, ns->ut,
-		ns->rhs, ns->a, ns->b, ns->rky, ns->J, ns->J + 3, ns->J + 6, ns->p };
+		ns->rhs, ns->a, ns->b, ns->rky, ns->p };
 	for (size_t k = 0; k < sizeof(all) / sizeof(all[0]); ++k)
 		for (int c = 0; c < 3; ++c)
 			hipFree(all[k][c]);
@@ -367,8 +366,6 @@ int ssx_ns_create(ssx_ns **out, ssx_ctx *c, const ssx_ns_params *prm)
 		for (int s = 0; s < 4 && rc == SSX_OK; ++s)
 			rc = nalloc(&ns->rkf[s][d], nt);
 	}
-	for (int k = 0; k < 9 && rc == SSX_OK; ++k)
-		rc = nalloc(&ns->J[k], nt);
 	/* zero histories (the element constructor's zeroed arrays) */
 	for (int l = 0; l < 3 && rc == SSX_OK; ++l) {
 		rc = ssxk_fill(c->stream, ns->p[l], 0.0, nt);
@@ -423,14 +420,10 @@ static int ns_double_curl(ssx_ns *ns, double *const u[3], double *const out[3])
 	void *st = ns->c->stream;
 	const ssx_level *L = &ns->c->lev[0];
 	const double *const *ti = (const double *const *) ns->ti;
-	TRYN(ssxk_ns_jac(st, ns->nt, ns->n, L->dmat, (const double *const *) u,
-			ns->J));
-	TRYN(ssxk_ns_curl(st, ns->nt, (const double *const *) ns->J, ti, NULL,
-			ns->a));
-	TRYN(ssxk_ns_jac(st, ns->nt, ns->n, L->dmat,
-			(const double *const *) ns->a, ns->J));
-	return ssxk_ns_curl(st, ns->nt, (const double *const *) ns->J, ti, L->mass,
-			out);
+	TRYN(ssxk_ns_curl(st, ns->nel, ns->n, L->dmat,
+			(const double *const *) u, ti, NULL, ns->a));
+	return ssxk_ns_curl(st, ns->nel, ns->n, L->dmat,
+			(const double *const *) ns->a, ti, L->mass, out);
 }
 
 /* U(t), the velocity history interpolated to time t with Lagrange weights,
@@ -605,11 +598,9 @@ int ssx_ns_step(ssx_ns *ns, ssx_stats stats[4])
 		/* DSS and inverse mass of each component */
 		TRYN(ns_inv_mass(ns, ns->b));
 		/* rhs = -dens/dt div u~ (weak), surface terms on Dirichlet faces */
-		TRYN(ssxk_ns_jac(st, nt, ns->n, L->dmat,
-				(const double *const *) ns->ut, ns->J));
-		TRYN(ssxk_ns_div(st, nt, (const double *const *) ns->J,
-				(const double *const *) ns->ti, L->mass, -ns->dens / dt,
-				ns->rhs[0]));
+		TRYN(ssxk_ns_div(st, ns->nel, ns->n, L->dmat,
+				(const double *const *) ns->ut, (const double *const *) ns->ti,
+				L->mass, -ns->dens / dt, ns->rhs[0]));
 		for (int d = 0; d < 3; ++d)
 			TRYN(ssxk_ns_surf(st, ns->nel, ns->n, L->bc, 1, ns->wn[d],
 					ns->b[d], ns->rhs[0]));
@@ -636,7 +627,7 @@ int ssx_ns_step(ssx_ns *ns, ssx_stats stats[4])
 	/* -- compute_velocity_rhs (navier_stokes.c:177-201) -- */
 	TRYN(ssxk_ns_mul3(st, nt, 1.0 / (dt * ns->visc),
 			(const double *const *) ns->ut, NULL, 0.0, ns->ut));
-	TRYN(ssxk_ns_grad(st, nt, ns->n, L->dmat, ns->p[0], L->mass,
+	TRYN(ssxk_ns_grad(st, ns->nel, ns->n, L->dmat, ns->p[0], L->mass,
 			(const double *const *) ns->ti, ns->b));
 	{
 		const double *ms[3] = { L->mass, L->mass, L->mass };

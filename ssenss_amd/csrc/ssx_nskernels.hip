@@ -30,130 +30,146 @@
 struct P3 { const double *p[3]; };
 struct M3 { double *p[3]; };
 struct P9 { const double *p[9]; };
-struct M9 { double *p[9]; };
 
 static inline unsigned ns_blocks(size_t n)
 {
 	return (unsigned) ((n + 255) / 256);
 }
 
-// reference derivative of u along direction d at node (k,j,i) of element
-// base `u` (n^3 block)
-__device__ __forceinline__ double dref(const double *__restrict__ u,
-		const double *__restrict__ dm, int n, int d, int k, int j, int i)
-{
-	double s = 0.0;
-	if (d == 0) {
-		const double *r = u + (k * n + j) * n;
-		for (int l = 0; l < n; ++l)
-			s += dm[i * n + l] * r[l];
-	} else if (d == 1) {
-		const double *r = u + k * n * n + i;
-		for (int l = 0; l < n; ++l)
-			s += dm[j * n + l] * r[l * n];
-	} else {
-		const double *r = u + j * n + i;
-		for (int l = 0; l < n; ++l)
-			s += dm[k * n + l] * r[l * n * n];
-	}
-	return s;
-}
+// The curl and the weak divergence of a field a, from its Jacobian J[3a+b] =
+// D_b a_a (compute_jacobian, deriv.c:68-79), in one launch:
+// curl (discrete_curl_operator, stokes.c:71-92): omega_c, for c = 0..2 and
+// xi-direction i = 0..2 in that loop order, += s_c (D_i u_k)(d xi_i/d x_l)
+// - s_c (D_i u_l)(d xi_i/d x_k) with k = (5-c)/2, l = (2-c)/2, s = (+1, -1,
+// +1); with mass, times w detJ (the test-function product of
+// double_curl_operator, stokes.c:94-105).
+// divergence (DIV; discrete_divergence_operator, stokes.c:52-69): sum_a sum_b
+// (D_b u_a)(d xi_b/d x_a) in that loop order, times w detJ, times `scale`.
+//
+// Bound by the 16 values (divergence: 14) a node that it moves: n = 10, 9.2
+// million nodes, 197 us at 6 TB/s.  A workgroup takes the elements that make
+// about 512 nodes, or one element, with the three fields and D in LDS, so
+// that a node's 9 n products read LDS; read from memory, with the Jacobian
+// stored between two launches, the curl took 826 + 300 us; now 225, the
+// divergence 1102 -> 221.
+template <int N>
+struct JacShape {
+	static constexpr int N3 = N * N * N;
+	static constexpr int E = N3 >= 512 ? 1 : 512 / N3;
+};
 
-// J[3a+b] = D_b a_a for three fields a_0..a_2 (compute_jacobian,
-// deriv.c:68-79)
+template <int N, bool DIV>
 __global__ void __launch_bounds__(256)
-k_ns_jac(long long nt, int n, const double *__restrict__ dm, P3 a, M9 out)
+k_ns_jac(int nel, const double *__restrict__ dm, P3 a, P9 ti,
+		const double *__restrict__ mass, double scale, M3 out)
 {
-	const long long q = (long long) blockIdx.x * 256 + threadIdx.x;
-	if (q >= nt)
-		return;
-	const int n3 = n * n * n;
-	const long long e = q / n3;
-	const int r = (int) (q - e * n3);
-	const int i = r % n, j = (r / n) % n, k = r / (n * n);
-	for (int f = 0; f < 3; ++f) {
-		const double *u = a.p[f] + e * n3;
-		for (int d = 0; d < 3; ++d)
-			out.p[3 * f + d][q] = dref(u, dm, n, d, k, j, i);
-	}
-}
-
-// curl from the Jacobian of u (discrete_curl_operator, stokes.c:71-92):
-// omega_c, for c = 0..2 and xi-direction i = 0..2 in that loop order,
-// += s_c (D_i u_k)(d xi_i/d x_l) - s_c (D_i u_l)(d xi_i/d x_k) with
-// k = (5-c)/2, l = (2-c)/2, s = (+1, -1, +1); with mass, times w detJ
-// (the test-function product of double_curl_operator, stokes.c:94-105)
-__global__ void __launch_bounds__(256)
-k_ns_curl(long long nt, P9 J, P9 ti, const double *__restrict__ mass,
-		M3 out)
-{
-	const long long q = (long long) blockIdx.x * 256 + threadIdx.x;
-	if (q >= nt)
-		return;
-	double jv[9], tv[9];
-	for (int a = 0; a < 9; ++a) {
-		jv[a] = J.p[a][q];
-		tv[a] = ti.p[a][q];
-	}
-	double om[3];
-	for (int i = 0; i < 3; ++i)
-		for (int c = 0; c < 3; ++c) {
-			const int k = (5 - c) / 2, l = (2 - c) / 2;
-			const double s = c == 1 ? -1.0 : 1.0;
-			const double t = s * jv[3 * k + i] * tv[3 * l + i];
-			om[c] = i == 0 ? t : t + om[c];
-			om[c] = -s * jv[3 * l + i] * tv[3 * k + i] + om[c];
-		}
+	constexpr int N3 = JacShape<N>::N3, E = JacShape<N>::E;
+	__shared__ double sa[3][E * N3], sd[N][N + 1];
+	const int e0 = blockIdx.x * E;
+	const int m = (nel - e0 < E ? nel - e0 : E) * N3;
+	const size_t b0 = (size_t) e0 * N3;
+	for (int q = threadIdx.x; q < N * N; q += 256)
+		sd[q / N][q % N] = dm[q];
+#pragma unroll
 	for (int c = 0; c < 3; ++c)
-		out.p[c][q] = mass ? om[c] * mass[q] : om[c];
-}
-
-// weak divergence (discrete_divergence_operator, stokes.c:52-69):
-// sum_a sum_b (D_b u_a)(d xi_b/d x_a) in that loop order, times w detJ,
-// times `scale`
-__global__ void __launch_bounds__(256)
-k_ns_div(long long nt, P9 J, P9 ti, const double *__restrict__ mass,
-		double scale, double *__restrict__ out)
-{
-	const long long q = (long long) blockIdx.x * 256 + threadIdx.x;
-	if (q >= nt)
-		return;
-	double s = 0.0;
-	for (int a = 0; a < 3; ++a)
-		for (int b = 0; b < 3; ++b) {
-			const double t = J.p[3 * a + b][q] * ti.p[3 * a + b][q];
-			s = (a + b == 0) ? t : t + s;
+		for (int q = threadIdx.x; q < m; q += 256)
+			sa[c][q] = a.p[c][b0 + q];
+	__syncthreads();
+	for (int q = threadIdx.x; q < m; q += 256) {
+		double tv[9];
+#pragma unroll
+		for (int b = 0; b < 9; ++b)
+			tv[b] = ti.p[b][b0 + q];
+		const double mv = mass ? mass[b0 + q] : 1.0;
+		const int i = q % N, j = (q / N) % N, k = (q / (N * N)) % N;
+		const int x0 = q - i, y0 = q - j * N, z0 = q - k * N * N;
+		double jv[9];
+#pragma unroll
+		for (int b = 0; b < 9; ++b)
+			jv[b] = 0.0;
+#pragma unroll
+		for (int l = 0; l < N; ++l) {
+			const double dx = sd[i][l], dy = sd[j][l], dz = sd[k][l];
+#pragma unroll
+			for (int c = 0; c < 3; ++c) {
+				jv[3 * c] += dx * sa[c][x0 + l];
+				jv[3 * c + 1] += dy * sa[c][y0 + l * N];
+				jv[3 * c + 2] += dz * sa[c][z0 + l * N * N];
+			}
 		}
-	out[q] = (s * mass[q]) * scale;
+		if (DIV) {
+			double s = jv[0] * tv[0];
+#pragma unroll
+			for (int b = 1; b < 9; ++b)
+				s = jv[b] * tv[b] + s;
+			out.p[0][b0 + q] = (s * mv) * scale;
+		} else {
+#pragma unroll
+			for (int c = 0; c < 3; ++c) {
+				const int kk = (5 - c) / 2, l = (2 - c) / 2;
+				const double s = c == 1 ? -1.0 : 1.0;
+				double om = 0.0;
+#pragma unroll
+				for (int b = 0; b < 3; ++b) {
+					const double t = s * jv[3 * kk + b] * tv[3 * l + b];
+					om = b == 0 ? t : t + om;
+					om = -s * jv[3 * l + b] * tv[3 * kk + b] + om;
+				}
+				out.p[c][b0 + q] = om * mv;
+			}
+		}
+	}
 }
 
 // weak gradient (discrete_gradient_operator, stokes.c:30-50): with
 // t = p w detJ and f_b = (d xi_b/d x_c) t, grad_c = -(D_xi^T f_0 +
 // D_eta^T f_1 + D_zeta^T f_2) (transpose_divergence, deriv.c:54-66)
+// Bound by the 14 values a node that it moves.  Laid out as k_ns_jac, one
+// component's three f_b in LDS at a time; read from memory by each of the 3 n
+// nodes that use it, it took 1626 us on 9.2 million nodes, n = 10; now 254.
+template <int N>
 __global__ void __launch_bounds__(256)
-k_ns_grad(long long nt, int n, const double *__restrict__ dm,
-		const double *__restrict__ p, const double *__restrict__ mass, P9 ti,
-		M3 out)
+k_ns_grad(int nel, const double *__restrict__ dm, const double *__restrict__ p,
+		const double *__restrict__ mass, P9 ti, M3 out)
 {
-	const long long q = (long long) blockIdx.x * 256 + threadIdx.x;
-	if (q >= nt)
-		return;
-	const int n3 = n * n * n;
-	const long long e = q / n3;
-	const int r = (int) (q - e * n3);
-	const int i = r % n, j = (r / n) % n, k = r / (n * n);
-	const long long b0 = e * n3;
+	constexpr int N3 = JacShape<N>::N3, E = JacShape<N>::E;
+	constexpr int R = (E * N3 + 255) / 256;
+	__shared__ double sf[3][E * N3], sd[N][N + 1];
+	const int e0 = blockIdx.x * E;
+	const int m = (nel - e0 < E ? nel - e0 : E) * N3;
+	const size_t b0 = (size_t) e0 * N3;
+	for (int q = threadIdx.x; q < N * N; q += 256)
+		sd[q % N][q / N] = dm[q];           // transposed: sd[i][l] = D_li
+	double t[R];
+#pragma unroll
+	for (int r = 0; r < R; ++r) {
+		const int q = threadIdx.x + 256 * r;
+		t[r] = q < m ? p[b0 + q] * mass[b0 + q] : 0.0;
+	}
 	for (int c = 0; c < 3; ++c) {
-		double sx = 0.0, sy = 0.0, sz = 0.0;
-		for (int l = 0; l < n; ++l) {
-			const long long qx = b0 + (k * n + j) * n + l;
-			const long long qy = b0 + (k * n + l) * n + i;
-			const long long qz = b0 + (l * n + j) * n + i;
-			sx += dm[l * n + i] * (ti.p[3 * c][qx] * (p[qx] * mass[qx]));
-			sy += dm[l * n + j] * (ti.p[3 * c + 1][qy] * (p[qy] * mass[qy]));
-			sz += dm[l * n + k] * (ti.p[3 * c + 2][qz] * (p[qz] * mass[qz]));
+#pragma unroll
+		for (int r = 0; r < R; ++r) {
+			const int q = threadIdx.x + 256 * r;
+			if (q < m) {
+#pragma unroll
+				for (int b = 0; b < 3; ++b)
+					sf[b][q] = ti.p[3 * c + b][b0 + q] * t[r];
+			}
 		}
-		out.p[c][q] = -((sx + sy) + sz);
+		__syncthreads();
+		for (int q = threadIdx.x; q < m; q += 256) {
+			const int i = q % N, j = (q / N) % N, k = (q / (N * N)) % N;
+			const int x0 = q - i, y0 = q - j * N, z0 = q - k * N * N;
+			double sx = 0.0, sy = 0.0, sz = 0.0;
+#pragma unroll
+			for (int l = 0; l < N; ++l) {
+				sx += sd[i][l] * sf[0][x0 + l];
+				sy += sd[j][l] * sf[1][y0 + l * N];
+				sz += sd[k][l] * sf[2][z0 + l * N * N];
+			}
+			out.p[c][b0 + q] = -((sx + sy) + sz);
+		}
+		__syncthreads();
 	}
 }
 
@@ -798,50 +814,52 @@ extern "C" int ssxk_ns_dss3(void *st, int *const grp[3],
 	return SSX_OK;
 }
 
-extern "C" int ssxk_ns_jac(void *st, size_t nt, int n, const double *dm,
-		const double *const a[3], double *const out[9])
+template <bool DIV>
+static int launch_jac(const char *name, void *st, int nel, int n,
+		const double *dm, const double *const a[3], const double *const ti[9],
+		const double *mass, double scale, M3 out)
 {
 	P3 pa = { { a[0], a[1], a[2] } };
-	M9 po;
+	P9 pt;
 	for (int k = 0; k < 9; ++k)
-		po.p[k] = out[k];
-	hipLaunchKernelGGL(k_ns_jac, dim3(ns_blocks(nt)), dim3(256), 0,
-			(hipStream_t) st, (long long) nt, n, dm, pa, po);
-	NS_LAUNCH("k_ns_jac");
+		pt.p[k] = ti[k];
+#define JCASE(N)                                                             \
+	case N:                                                              \
+		hipLaunchKernelGGL((k_ns_jac<N, DIV>), dim3((unsigned) ((nel     \
+				+ JacShape<N>::E - 1) / JacShape<N>::E)), dim3(256), 0, \
+				(hipStream_t) st, nel, dm, pa, pt, mass, scale, out); \
+		break;
+	switch (n) {
+	JCASE(2) JCASE(3) JCASE(4) JCASE(5) JCASE(6) JCASE(7) JCASE(8)
+	JCASE(9) JCASE(10)
+	default:
+		ssx_set_error("%s: %d points per direction (2..10)", name, n);
+		return SSX_EINVAL;
+	}
+#undef JCASE
+	NS_LAUNCH(name);
 	return SSX_OK;
 }
 
-extern "C" int ssxk_ns_curl(void *st, size_t nt, const double *const J[9],
-		const double *const ti[9], const double *mass, double *const out[3])
+extern "C" int ssxk_ns_curl(void *st, int nel, int n, const double *dm,
+		const double *const a[3], const double *const ti[9],
+		const double *mass, double *const out[3])
 {
-	P9 pj, pt;
-	for (int k = 0; k < 9; ++k) {
-		pj.p[k] = J[k];
-		pt.p[k] = ti[k];
-	}
 	M3 po = { { out[0], out[1], out[2] } };
-	hipLaunchKernelGGL(k_ns_curl, dim3(ns_blocks(nt)), dim3(256), 0,
-			(hipStream_t) st, (long long) nt, pj, pt, mass, po);
-	NS_LAUNCH("k_ns_curl");
-	return SSX_OK;
+	return launch_jac<false>("ssxk_ns_curl", st, nel, n, dm, a, ti, mass, 1.0,
+			po);
 }
 
-extern "C" int ssxk_ns_div(void *st, size_t nt, const double *const J[9],
-		const double *const ti[9], const double *mass, double scale,
-		double *out)
+extern "C" int ssxk_ns_div(void *st, int nel, int n, const double *dm,
+		const double *const a[3], const double *const ti[9],
+		const double *mass, double scale, double *out)
 {
-	P9 pj, pt;
-	for (int k = 0; k < 9; ++k) {
-		pj.p[k] = J[k];
-		pt.p[k] = ti[k];
-	}
-	hipLaunchKernelGGL(k_ns_div, dim3(ns_blocks(nt)), dim3(256), 0,
-			(hipStream_t) st, (long long) nt, pj, pt, mass, scale, out);
-	NS_LAUNCH("k_ns_div");
-	return SSX_OK;
+	M3 po = { { out, nullptr, nullptr } };
+	return launch_jac<true>("ssxk_ns_div", st, nel, n, dm, a, ti, mass, scale,
+			po);
 }
 
-extern "C" int ssxk_ns_grad(void *st, size_t nt, int n, const double *dm,
+extern "C" int ssxk_ns_grad(void *st, int nel, int n, const double *dm,
 		const double *p, const double *mass, const double *const ti[9],
 		double *const out[3])
 {
@@ -849,8 +867,20 @@ extern "C" int ssxk_ns_grad(void *st, size_t nt, int n, const double *dm,
 	for (int k = 0; k < 9; ++k)
 		pt.p[k] = ti[k];
 	M3 po = { { out[0], out[1], out[2] } };
-	hipLaunchKernelGGL(k_ns_grad, dim3(ns_blocks(nt)), dim3(256), 0,
-			(hipStream_t) st, (long long) nt, n, dm, p, mass, pt, po);
+#define GCASE(N)                                                             \
+	case N:                                                              \
+		hipLaunchKernelGGL(k_ns_grad<N>, dim3((unsigned) ((nel           \
+				+ JacShape<N>::E - 1) / JacShape<N>::E)), dim3(256), 0, \
+				(hipStream_t) st, nel, dm, p, mass, pt, po); \
+		break;
+	switch (n) {
+	GCASE(2) GCASE(3) GCASE(4) GCASE(5) GCASE(6) GCASE(7) GCASE(8)
+	GCASE(9) GCASE(10)
+	default:
+		ssx_set_error("ssxk_ns_grad: %d points per direction (2..10)", n);
+		return SSX_EINVAL;
+	}
+#undef GCASE
 	NS_LAUNCH("k_ns_grad");
 	return SSX_OK;
 }
