@@ -2384,8 +2384,9 @@ int ssx_tracers_step_host(ssx_ctx *c, const ssx_particles *h, double t_now,
 /* ------------------------------------------------------------------ */
 
 /* average time in microseconds of `reps` Poisson operator launches of
- * variant v on level l in precision prec, on the context's stream */
-static int time_ax(ssx_ctx *c, int l, int prec, int v, int reps,
+ * variant v on level l in precision prec, on the context's stream; team:
+ * the team kernel where the operator runs the matrix kernel */
+static int time_ax(ssx_ctx *c, int l, int prec, int v, int team, int reps,
 		double *us)
 {
 	ssx_level *L = &c->lev[l];
@@ -2399,7 +2400,10 @@ static int time_ax(ssx_ctx *c, int l, int prec, int v, int reps,
 			rc = SSX_EHIP;
 		if (rc)
 			break;
-		if (prec == SSX_PREC_FP64)
+		if (team)
+			rc = ssxk_ax_team(c->stream, L->n, v, c->nel, L->p, L->ap, L->gf,
+					L->mass, L->dmat, c->lambda, L->bc, c->part);
+		else if (prec == SSX_PREC_FP64)
 			rc = ssxk_ax(c->stream, L->n, v, c->nel, SSX_OP_POISSON, L->p,
 					L->ap, L->gf, L->mass, L->dmat, c->lambda, L->bc, 1, NULL,
 					c->part);
@@ -2441,16 +2445,30 @@ int ssx_autotune(ssx_ctx *c, int prec_mask)
 			/* enough launches for about a millisecond of work */
 			const int reps = L->ntot > (1 << 22) ? 5
 				: L->ntot > (1 << 18) ? 20 : 50;
+			const int matrix = prec == SSX_PREC_FP64
+				&& ssxk_ax_matrix(L->n, c->nel);
 			double best = 0.0;
 			int bv = 0;
 			for (int v = 0; v < SSX_AX_NVARIANTS; ++v) {
 				double us;
-				TRY(time_ax(c, l, prec, v, reps, &us));
+				TRY(time_ax(c, l, prec, v, matrix, reps, &us));
 				c->ax_us[l][prec][v] = us;
 				if (v == 0 || us < best) {
 					best = us;
 					bv = v;
 				}
+			}
+			/* The matrix kernel has of the shape only the streaming hint
+			 * (bit 1); the other bits are the batched operator's, which is
+			 * the team kernel at these sizes too, so they come from its
+			 * times above and the hint from the matrix kernel's. */
+			if (matrix) {
+				double us[2];
+				for (int h = 0; h < 2; ++h)
+					TRY(time_ax(c, l, prec, 2 * h, 0, reps, us + h));
+				for (int v = 0; v < SSX_AX_NVARIANTS; ++v)
+					c->ax_us[l][prec][v] = us[(v >> 1) & 1];
+				bv = us[1] < us[0] ? bv | 2 : bv & ~2;
 			}
 			L->axv[prec] = bv;
 		}

@@ -308,6 +308,12 @@ int ssxk_ax(void *stream, int n, int v, int nel, int op, const double *u,
 		double *au, const double *gf, const double *mass,
 		const double *dmat, double lambda, const int *bc, int apply_mask,
 		const int *done, double *part);
+/* the FP64 operator runs the matrix kernel at these sizes; the team kernel
+ * there (Poisson, masked), n = 9..12, for ranking the batch's shapes */
+int ssxk_ax_matrix(int n, int nel);
+int ssxk_ax_team(void *stream, int n, int v, int nel, const double *u,
+		double *au, const double *gf, const double *mass,
+		const double *dmat, double lambda, const int *bc, double *part);
 /* A reduction of the fused CG replayed by the kernel that needs it instead
  * of a launch of its own (part != NULL): every workgroup sums the cnt
  * partials exactly as ssxk_cg_reduce does and forms the same scalars;

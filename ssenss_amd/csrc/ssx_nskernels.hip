@@ -637,7 +637,7 @@ k_ns_mul3(long long nt, double alpha, P3 x, P3 w, double beta, M3 z)
 // Bound by the T + 1 (+ 4) values it moves (T = 3 with STAGE: 311 us on 9.2
 // million nodes, 5.7 TB/s).  The stage had 13 launches: three copies, three
 // fills, two sums read and written in place, one DSS a component, the
-// inverse mass; 2 to 5 us each on 512 elements of 8 points, 0.83 ms
+// inverse mass; 2 to 5 us each on 64 elements of 8 points, 0.83 ms
 // together on the 9.2 million nodes.  Now this, the operator and one DSS,
 // and a velocity formed once for the stages at one time: 0.43 ms.
 struct RkTerms {
