@@ -1077,12 +1077,16 @@ static int cg_level_fused(ssx_ctx *c, int l, int op, int var, double *f,
 		max_iter, pres, flags, eps_dev, (double) L->nunique };
 	int launched = 0;
 	int chunk = c->cg_hint[l] > 0 ? c->cg_hint[l] + 1 : 8;
+	/* the last workgroups of the DSS and the update form the scalars; a
+	 * level without a shared node has no DSS launch and iterates as without
+	 * the option */
+	const int fused_red = c->fused_red && nbd > 0;
 	/* the solution step u += alpha p of each iteration is taken by the
 	 * next operator launch, from its load of p; the last one by a flush */
-	const int defer = !c->fused_red;
+	const int defer = !fused_red;
 	/* the two reductions of an iteration replayed by the kernels that need
 	 * them (two launches an iteration); the chunk's last one is a launch */
-	const int gather = c->gather_upd && L->gP > 0 && !c->fused_red;
+	const int gather = c->gather_upd && L->gP > 0 && !fused_red;
 	const int replay = gather && c->nel <= SSX_REPLAY_NEL;
 	double *pu = replay ? c->part + c->nel : c->part;
 	const int nbu = gather ? ssxk_cg_update_blocks(nt) : 0;
@@ -1108,14 +1112,14 @@ static int cg_level_fused(ssx_ctx *c, int l, int op, int var, double *f,
 						L->mass, L->dmat, c->lambda, L->bc, !pres, flags,
 						c->part, defer ? u : NULL, o + CG_ALPHA,
 						replay && k > 0 ? &rb : NULL));
-			if (c->fused_red && nbd > 0) {
+			if (fused_red) {
 				TRY(ssxk_dss_all_red(st, L->grp, L->ngrp, ap, NULL, NULL,
 						flags, &lr0));
 				TRY(ssxk_cg_update_red(st, nt, c->scal, o + CG_ALPHA, p, ap,
 						u, r, z, dinv, L->scale, pres, c->part, flags, &lr1));
 				continue;
 			}
-			if (c->gather_upd && L->gP > 0) {
+			if (gather) {
 				/* alpha needs only the operator's partials; the
 				 * update then assembles Ap as it reads it */
 				if (!replay)
@@ -1389,8 +1393,8 @@ static int cg_level_lp(ssx_ctx *c, int l, int op, int var, float *f,
 	 * factors 0.183 -> 0.185 s, bit-identical results) */
 	const int defer = 0;
 	/* as cg_level_fused: reductions replayed on small levels */
-	const int gather = c->gather_upd && L->gP > 0
-		&& !(c->fused_red && ssxk_dss_blocks(L->ngrp) > 0);
+	const int fused_red = c->fused_red && ssxk_dss_blocks(L->ngrp) > 0;
+	const int gather = c->gather_upd && L->gP > 0 && !fused_red;
 	const int replay = gather && c->nel <= SSX_REPLAY_NEL_LP;
 	double *pu = replay ? c->part + c->nel : c->part;
 	const int nbu = gather ? ssxk_cg_update_blocks(nt) : 0;
@@ -1412,7 +1416,7 @@ static int cg_level_lp(ssx_ctx *c, int l, int op, int var, float *f,
 					L->gf_lp, L->mass_lp, L->dmat_lp, c->lambda, L->bc, !pres,
 					flags, c->part, defer ? u : NULL, o + CG_ALPHA,
 					replay ? &rb : NULL));
-		if (c->fused_red && ssxk_dss_blocks(L->ngrp) > 0) {
+		if (fused_red) {
 			const ssx_lastred lr0 = { c->redctr, c->part, nba, c->scal, o,
 				max_iter, pres, flags, eps, (double) L->nunique };
 			const ssx_lastred lr1 = { c->redctr + 1, c->part, SSX_NPART,
@@ -1423,7 +1427,7 @@ static int cg_level_lp(ssx_ctx *c, int l, int op, int var, float *f,
 					r, z, dinv, L->scale_lp, pres, c->part, flags, &lr1));
 			continue;
 		}
-		if (c->gather_upd && L->gP > 0) {
+		if (gather) {
 			if (!replay)
 				TRY(ssxk_cg_reduce(st, 0, c->part, nba, c->scal, o, flags,
 						eps, max_iter, L->nunique, pres));
