@@ -74,6 +74,15 @@ struct PUpd {
 // of a stopped solve then loads one element a workgroup for nothing)
 #define SSX_LATE_FLAG_GRID 2048
 
+// The done flag is read late.  A launch that replays the stopping test always
+// does: its workgroup 0 may set the flag (rp.flags aliases done) while others
+// still read it, so two wavefronts of one workgroup can see different values;
+// the exit then hangs on lane 0's alone, through LDS (replay_beta).
+__device__ __forceinline__ bool ax_late(int pu, const ssx_replay &rp)
+{
+	return pu >= 1 && (rp.part || gridDim.x <= SSX_LATE_FLAG_GRID);
+}
+
 // the scalars of the fused direction update
 struct AxScal {
 	double b, c, a;              // beta, null-space constant, alpha
@@ -121,7 +130,8 @@ __device__ __forceinline__ void replay_sums(const double *__restrict__ part,
 // beta, the null-space constant and the stopping test of the previous
 // iteration (cg_scalars1) formed by every workgroup from the update's
 // partials; workgroup 0 stores them.  Every lane of the workgroup calls it;
-// dn: the solve had stopped before this launch (nothing is stored).
+// dn: the solve had stopped before this launch (nothing is stored; lane 0's
+// value counts).
 template <int BLOCK>
 __device__ __forceinline__ AxScal replay_beta(const ssx_replay &rp, int dn)
 {
@@ -441,7 +451,7 @@ k_ax(int nel, const T *__restrict__ u, T *__restrict__ au,
 		const G *__restrict__ gf, const T *__restrict__ mass,
 		const T *__restrict__ dmat, T lambda,
 		const int *__restrict__ bc, int apply_mask,
-		const int *__restrict__ done, double *__restrict__ part,
+		const int *done, double *__restrict__ part,
 		const T *__restrict__ zin, T *__restrict__ pio,
 		const double *__restrict__ scal, int ib, int ic,
 		T *__restrict__ uio, int ia, ssx_replay rp)
@@ -449,7 +459,7 @@ k_ax(int nel, const T *__restrict__ u, T *__restrict__ au,
 	// Solver already converged: no-op.  A small launch, which lasts a few
 	// trips to memory, reads the flag along with its operands instead of
 	// one trip ahead of them (PU: after the element's loads).
-	const bool late = PU >= 1 && gridDim.x <= SSX_LATE_FLAG_GRID;
+	const bool late = ax_late(PU, rp);
 	const int dn = done ? *done : 0;
 	if (!late && dn)
 		return;

@@ -330,13 +330,13 @@ k_axm(const double *__restrict__ u, double *__restrict__ au,
 		const double *__restrict__ gf, const double *__restrict__ mass,
 		const double *__restrict__ dmat, double lambda,
 		const int *__restrict__ bc, int apply_mask,
-		const int *__restrict__ done, double *__restrict__ part,
+		const int *done, double *__restrict__ part,
 		const double *__restrict__ zin, double *__restrict__ pio,
 		const double *__restrict__ scal, int ib, int ic,
 		double *__restrict__ uio, int ia, ssx_replay rp)
 {
 	__shared__ double sm[AxmShape<N>::LDS];
-	const bool late = PU >= 1 && gridDim.x <= SSX_LATE_FLAG_GRID;
+	const bool late = ax_late(PU, rp);
 	const int dn = done ? *done : 0;     // converged: no-op (as k_ax)
 	if (!late && dn)
 		return;

@@ -7,8 +7,9 @@ The replay sums in the order of a 1024-lane reduction, so its edges are the
 numbers of partials: elements below, at and above 1024 (a virtual lane's
 second partial), the largest level that replays (FP64 1024, FP32 4096
 elements) and the first that does not; workgroups smaller than a wavefront
-(n = 3, 5, 6, 7 under the one-wave launch shapes) and of several; the
-pressure's four sums; a solve that stops in the middle of a chunk of
+(n = 3, 5, 6, 7 under the one-wave launch shapes) and of several, below and
+above the 2048 workgroups up to which every launch reads the done flag late
+(a replaying one always does); the pressure's four sums; a solve that stops in the middle of a chunk of
 launches and one stopped by its iteration limit."""
 import numpy as np
 import pytest
@@ -99,3 +100,30 @@ def test_replayed_reductions_by_workgroup(n, variant):
         return res
     print(f"[gpu] replay n={n} variant {variant}", flush=True)
     _same(*_pair(mesh, run, variant))
+
+
+@pytest.mark.parametrize("dims", [(8, 16, 16), (13, 13, 13)])
+def test_replayed_stop_by_grid(dims):
+    """One team of two wavefronts a workgroup (n = 9, one-wave shape): 2048
+    and 2197 workgroups, stopped before the smoother's last iteration."""
+    mesh = box_mesh(9, dims, deform=1, amp=0.05, dt=0.1, visc=0.1)
+
+    def run(ctx):
+        res = []
+        for prec in (S.PREC_FP32, S.PREC_BF16):
+            ctx.set_option(S.OPT_SMOOTHER_PRECISION, prec)
+            zs = []
+            for eps in (1e-12, 0.05):   # the first call picks a shape
+                f = _rhs(ctx, 6)
+                z = torch.zeros_like(f)
+                ctx.mask(0, S.X_VELOCITY, f)
+                norm = float(np.sqrt(ctx.dot(0, f, f)))
+                ctx.mg_precon(S.OP_HELMHOLTZ, S.X_VELOCITY, eps * norm, f, z)
+                zs.append(z)
+                ctx.set_ax_variant(0, prec, 1)
+            assert not torch.equal(*zs)         # it did stop early
+            res += zs
+        ctx.set_option(S.OPT_SMOOTHER_PRECISION, S.PREC_FP64)
+        return res
+    print(f"[gpu] replayed stop {dims}", flush=True)
+    _same(*_pair(mesh, run))
