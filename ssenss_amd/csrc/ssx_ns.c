@@ -60,6 +60,7 @@ int ssxk_ns_grad(void *st, int nel, int n, const double *dm,
 int ssxk_ns_conv(void *st, int nel, int n, const double *prol,
 		const double *dm, const double *const u[3], const double *const v[3],
 		const double *geo, double *const out[3]);
+int ssxk_ns_conv_ready(int n);
 int ssxk_ns_surf(void *st, int nel, int n, const int *bc, int dirichlet,
 		const double *wn, const double *g, double *f);
 int ssxk_ns_zero_dir(void *st, size_t nt, int n, const int *bc,
@@ -330,6 +331,8 @@ int ssx_ns_create(ssx_ns **out, ssx_ctx *c, const ssx_ns_params *prm)
 				"not (11/6)/(dt visc) = %g", c->lambda, lam);
 		return SSX_EINVAL;
 	}
+	/* refused here, not in the middle of a step */
+	TRYN(ssxk_ns_conv_ready(n));
 	ssx_ns *ns = calloc(1, sizeof(*ns));
 	if (!ns)
 		return SSX_ENOMEM;

@@ -508,6 +508,21 @@ k_ns_conv(const double *__restrict__ prol, const double *__restrict__ dm,
 		[&](int f, int l) { return (f == 0 ? o0 : f == 1 ? o1 : o2) + l; });
 }
 
+// the element's LDS granted to the kernel on the current device
+template <int N>
+static int conv_lds(void)
+{
+	constexpr int NC = (3 * N) / 2;
+	using S = ConvShape<N, NC>;
+	if (hipFuncSetAttribute((const void *) k_ns_conv<N, NC>,
+			hipFuncAttributeMaxDynamicSharedMemorySize, (int) S::BYTES)
+			!= hipSuccess) {
+		ssx_set_error("k_ns_conv: %zu bytes of LDS refused", S::BYTES);
+		return SSX_EHIP;
+	}
+	return SSX_OK;
+}
+
 template <int N>
 static int launch_conv(hipStream_t st, int nel, const double *prol,
 		const double *dm, const P3 &u, const P3 &v, const double *geo,
@@ -516,12 +531,9 @@ static int launch_conv(hipStream_t st, int nel, const double *prol,
 	constexpr int NC = (3 * N) / 2;
 	using S = ConvShape<N, NC>;
 	static_assert(S::W <= 16 && S::BYTES <= 160 * 1024, "element too large");
-	if (hipFuncSetAttribute((const void *) k_ns_conv<N, NC>,
-			hipFuncAttributeMaxDynamicSharedMemorySize, (int) S::BYTES)
-			!= hipSuccess) {
-		ssx_set_error("k_ns_conv: %zu bytes of LDS refused", S::BYTES);
-		return SSX_EHIP;
-	}
+	const int rc = conv_lds<N>();
+	if (rc != SSX_OK)
+		return rc;
 	hipLaunchKernelGGL((k_ns_conv<N, NC>), dim3(nel), dim3(64 * S::W),
 			S::BYTES, st, prol, dm, u, v, geo, out);
 	return SSX_OK;
@@ -957,4 +969,31 @@ extern "C" int ssxk_ns_mul3(void *st, size_t nt, double alpha,
 			(hipStream_t) st, (long long) nt, alpha, px, pw, beta, pz);
 	NS_LAUNCH("k_ns_mul3");
 	return SSX_OK;
+}
+
+// whether the current device can run the convection operator at n points: a
+// workgroup's LDS (162,512 bytes at n = 10) within its limit, and granted
+extern "C" int ssxk_ns_conv_ready(int n)
+{
+	int dev = 0, lim = 0;
+	if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&lim,
+			hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess) {
+		ssx_set_error("k_ns_conv: no device to run on");
+		return SSX_EHIP;
+	}
+	size_t need = 0;
+	int rc = SSX_OK;
+	switch (n) {
+#define CASE(NN) case NN: need = ConvShape<NN, (3 * NN) / 2>::BYTES; \
+		rc = need <= (size_t) lim ? conv_lds<NN>() : SSX_EHIP; break;
+	CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(9) CASE(10)
+#undef CASE
+	default:
+		ssx_set_error("k_ns_conv: n = %d unsupported", n);
+		return SSX_EINVAL;
+	}
+	if (need > (size_t) lim)
+		ssx_set_error("k_ns_conv: n = %d needs %zu bytes of LDS, the device "
+				"has %d", n, need, lim);
+	return rc;
 }
