@@ -1007,6 +1007,38 @@ int ssx_cg_start(ssx_ctx *c, int l, int op, int var, double *f,
 #define RDZ_SLOT(k) ((k) < 0 || (k) % 2 == 0 ? CG_RDZ : CG_RDZ1)
 
 /*
+ * Whether a level's CG replays its reductions (lp: FP32 fields, FP32 or BF16
+ * factors) instead of launching them.  A launch costs 4.3 us and its gap, an
+ * iteration has two.  A replay costs a few microseconds (up to 1024 partials
+ * a quantity from memory, and one an element for alpha) as long as every
+ * workgroup has its slot at once; beyond that it comes round after round, so
+ * the limit falls with the wavefronts a workgroup has and the registers they
+ * take: 1 or 2 wavefronts up to n = 11, 3 and 4 from 12 on, 9 in the FP64
+ * matrix kernel of n = 12, whose factors wait for the replay.  us, launches /
+ * replayed:
+ *   FP64 CG iteration.  1000 elements: n = 3 16.8 / 14.2, 5 19.0 / 16.3, 8
+ *   26.5 / 25.7, 9 36.2 / 34.8, 10 43.9 / 39.0, 11 51.2 / 48.4; 2744: n = 3
+ *   18.0 / 16.0, 8 47.1 / 49.7, 10 90 / 97.  n = 13 512: 48.4 / 47.8, 729:
+ *   68.5 / 71.1; n = 14 512: 71.2 / 71.1, 1000: 126.6 / 128.6; n = 15 512: 63.9
+ *   / 62.9, 729: 96.4 / 99.9.  n = 12 64: 21.0 / 19.8, 125: 22.3 / 22.6, 1000:
+ *   62.4 / 69.1; n = 16 27: 37.5 / 36.1, 64: 39.5 / 40.1, 1000: 161 / 177.
+ *   FP32 V-cycle (the finest level's reductions from n = 9 on, every level's
+ *   below).  4096 elements: n = 5 763 / 742, 8 1158 / 1100, 9 1668 / 1657, 10
+ *   1913 / 1881, 11 2375 / 2448, 12 3030 / 3200; 5832: n = 5 852 / 900, 8 1361
+ *   / 1485.  n = 11 1728: 1496 / 1492; n = 12 1331: 1529 / 1523, 2744: 2214 /
+ *   2172; n = 13 1000: 1464 / 1462, 2744: 2719 / 2832; n = 15 1000: 1806 /
+ *   1800, 1728: 2675 / 2723; n = 16 216: 1164 / 1152, 512: 1407 / 1410, 1000:
+ *   2082 / 2142.
+ */
+static int replays(int n, int nel, int lp)
+{
+	if (lp)
+		return nel <= (n <= 10 ? 4096 : n <= 12 ? 2048 : n <= 15 ? 1024
+				: 256);
+	return nel <= (n <= 11 ? 1024 : n == 12 ? 64 : n <= 15 ? 512 : 32);
+}
+
+/*
  * The same iteration fused: Ax (from the second iteration on with the
  * direction update p = (z - c) + beta p of the previous one) and the sum of
  * p (A_e p) over all local copies, which for p equal on the copies of each
@@ -1087,7 +1119,7 @@ static int cg_level_fused(ssx_ctx *c, int l, int op, int var, double *f,
 	/* the two reductions of an iteration replayed by the kernels that need
 	 * them (two launches an iteration); the chunk's last one is a launch */
 	const int gather = c->gather_upd && L->gP > 0 && !fused_red;
-	const int replay = gather && c->nel <= SSX_REPLAY_NEL;
+	const int replay = gather && replays(L->n, c->nel, 0);
 	double *pu = replay ? c->part + c->nel : c->part;
 	const int nbu = gather ? ssxk_cg_update_blocks(nt) : 0;
 	for (;;) {
@@ -1395,7 +1427,7 @@ static int cg_level_lp(ssx_ctx *c, int l, int op, int var, float *f,
 	/* as cg_level_fused: reductions replayed on small levels */
 	const int fused_red = c->fused_red && ssxk_dss_blocks(L->ngrp) > 0;
 	const int gather = c->gather_upd && L->gP > 0 && !fused_red;
-	const int replay = gather && c->nel <= SSX_REPLAY_NEL_LP;
+	const int replay = gather && replays(L->n, c->nel, 1);
 	double *pu = replay ? c->part + c->nel : c->part;
 	const int nbu = gather ? ssxk_cg_update_blocks(nt) : 0;
 	for (int k = 0; k < max_iter; ++k) {

@@ -328,18 +328,6 @@ typedef struct ssx_replay {
 	int *flags;
 	double eps, nunique;
 } ssx_replay;
-/* Most elements of a level whose CG replays its reductions (FP64; FP32
- * fields).  A replay costs the operator 3.6 us and the update 2.4 us where
- * every workgroup has its slot at once, a launch 4.3 us and its gap.  The
- * FP64 operator's registers leave 8 wavefronts a CU, so past about a
- * thousand elements of two or more wavefronts the replay comes round
- * after round.  Measured per CG iteration, launches / replayed: FP64 n = 8
- * 64 elements 19.3 / 16.2 us, 1000: 26.6 / 25.3, 4096: 59.9 / 70.6, n = 12
- * 216: 32.7 / 30.7, 1728: 114.5 / 119.1; FP32 V-cycle n = 8 64: 635 / 508
- * us, 4096: 1169 / 1082, n = 12 1728: 1813 / 1776, n = 8 8000 (all
- * replayed): 1646 / 1845. */
-#define SSX_REPLAY_NEL 1024
-#define SSX_REPLAY_NEL_LP 4096
 /* ssxk_ax of the new CG direction: p = (z - scal[ic]) + scal[ib] p
  * (ic < 0: no null-space constant), masked where apply_mask, written back
  * to p, and ap = A p -- the k_cg_pupdate of the previous iteration fused

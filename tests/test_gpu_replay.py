@@ -5,8 +5,8 @@ same order): bit-identical solutions and iteration counts.
 
 The replay sums in the order of a 1024-lane reduction, so its edges are the
 numbers of partials: elements below, at and above 1024 (a virtual lane's
-second partial), the largest level that replays (FP64 1024, FP32 4096
-elements) and the first that does not; workgroups smaller than a wavefront
+second partial), the largest level that replays and the first that does not
+(up to n = 11 FP64 1024 and, to n = 10, FP32 4096 elements; fewer above); workgroups smaller than a wavefront
 (n = 3, 5, 6, 7 under the one-wave launch shapes) and of several, below and
 above the 2048 workgroups up to which every launch reads the done flag late
 (a replaying one always does); the pressure's four sums; a solve that stops in the middle of a chunk of
@@ -127,3 +127,12 @@ def test_replayed_stop_by_grid(dims):
         return res
     print(f"[gpu] replayed stop {dims}", flush=True)
     _same(*_pair(mesh, run))
+
+
+@pytest.mark.parametrize("n,dims", [
+    (12, (4, 4, 4)), (12, (2, 3, 11)), (13, (8, 8, 8)), (13, (9, 19, 3)),
+    (16, (4, 4, 2)), (16, (4, 3, 3)), (16, (16, 4, 4)), (16, (2, 3, 43))])
+def test_replayed_reductions_at_high_order(n, dims):
+    """The largest level that replays and one just past it: FP64 n = 12 (64 /
+    66 elements), 13 (512 / 513), 16 (32 / 36), FP32 n = 16 (256 / 258)."""
+    test_replayed_reductions_by_element_count(n, dims)
