@@ -2489,6 +2489,8 @@ int ssx_autotune(ssx_ctx *c, int prec_mask)
 				double us;
 				TRY(time_ax(c, l, prec, v, matrix, reps, &us));
 				c->ax_us[l][prec][v] = us;
+				if (matrix)
+					c->team_us[l][v] = us;
 				if (v == 0 || us < best) {
 					best = us;
 					bv = v;
@@ -2521,6 +2523,16 @@ int ssx_ax_variant(const ssx_ctx *c, int l, int prec,
 		for (int v = 0; v < SSX_AX_NVARIANTS; ++v)
 			us[v] = c->ax_us[l][prec][v];
 	return c->lev[l].axv[prec];
+}
+
+int ssx_ax_team_times(const ssx_ctx *c, int l, double us[SSX_AX_NVARIANTS])
+{
+	if (!c || l < 0 || l >= c->nlev
+			|| !ssxk_ax_matrix(c->lev[l].n, c->nel))
+		return 0;
+	for (int v = 0; v < SSX_AX_NVARIANTS; ++v)
+		us[v] = c->team_us[l][v];
+	return 1;
 }
 
 int ssx_set_ax_variant(ssx_ctx *c, int l, int prec, int v)

@@ -155,6 +155,8 @@ struct ssx_ctx {
 	long p_pass_np;              /* particles of the last pass-by-pass step */
 	long long cnt[4];
 	double ax_us[SSX_LMAX][3][SSX_AX_NVARIANTS];  /* autotuner timings  */
+	double team_us[SSX_LMAX][SSX_AX_NVARIANTS];   /* the team kernel's,
+	                                where the FP64 operator is the matrix one */
 };
 
 /* ---- sparse direct solver (ssx_sdirect.c, ssx_sdkernels.hip) ---- */
@@ -311,6 +313,10 @@ int ssxk_ax(void *stream, int n, int v, int nel, int op, const double *u,
 /* the FP64 operator runs the matrix kernel at these sizes; the team kernel
  * there (Poisson, masked), n = 9..12, for ranking the batch's shapes */
 int ssxk_ax_matrix(int n, int nel);
+/* the autotuner's times of the team kernel's shapes on level l, by which it
+ * picked the bits of the batch's shape; returns 0 where the operator is the
+ * team kernel itself (ssx_ax_variant has them) */
+int ssx_ax_team_times(const ssx_ctx *c, int l, double us[SSX_AX_NVARIANTS]);
 int ssxk_ax_team(void *stream, int n, int v, int nel, const double *u,
 		double *au, const double *gf, const double *mass,
 		const double *dmat, double lambda, const int *bc, double *part);
