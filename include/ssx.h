@@ -179,8 +179,8 @@ int ssx_set_diag_choice(ssx_ctx *ctx, int choice);
 #define SSX_OPT_SMOOTHER_PRECISION 2
 /* SSX_OPT_PERSISTENT_CG: 1 runs the fused CG of every multigrid
  * level with n <= 4 (the coarse levels) as one cooperative launch with
- * grid-wide barriers instead of six launches per iteration; 0 keeps the
- * per-iteration launches (default); a value 2..1024 also fixes the number of
+ * grid-wide barriers instead of two to four launches per iteration; 0 keeps
+ * the per-iteration launches (default); a value 2..1024 also fixes the number of
  * workgroups of that launch (default: as many as the device keeps
  * co-resident).  Same algorithm and stopping test; inner products are
  * summed in a different fixed order. */
@@ -191,10 +191,12 @@ int ssx_set_diag_choice(ssx_ctx *ctx, int choice);
 #define SSX_OPT_LP_COARSE_RTOL 4
 /* SSX_OPT_FUSED_REDUCE: 1 lets the last workgroup of the DSS and of the
  * update kernel form alpha and beta (three launches per fused CG
- * iteration); 0 (default) uses separate single-workgroup reductions
- * (five).  Same summation order: bit-identical results.  Off by default:
- * every workgroup's device-scope release (an L2 write-back per XCD) costs
- * more than the two launches it saves. */
+ * iteration); 0 (default) uses separate single-workgroup reductions with
+ * the DSS inside the update (four launches), on small levels replayed by
+ * the kernels that need them (two).  A level without a shared node has no
+ * DSS launch and iterates as with 0.  Same summation order: bit-identical
+ * results.  Off by default: every workgroup's device-scope release (an L2
+ * write-back per XCD) costs more than the launches it saves. */
 #define SSX_OPT_FUSED_REDUCE 5
 /* SSX_OPT_COARSE_ASSEMBLED: 1 (default) runs the p-multigrid coarsest-level
  * Jacobi-PCG over unique nodes with the level's operator assembled once

@@ -1402,7 +1402,7 @@ int ssx_cg_start_lp(ssx_ctx *c, int l, int op, int var, float *f,
 	return ssxk_reduce(st, part, 0, scal, o + CG_RDZ);
 }
 
-/* conjugate_gradient (solver.c:33-81) in FP32 storage: the fused six-kernel
+/* conjugate_gradient (solver.c:33-81) in FP32 storage: the fused
  * iteration of cg_level_fused with FP64 scalars and inner products */
 static int cg_level_lp(ssx_ctx *c, int l, int op, int var, float *f,
 		float *u, double eps, int max_iter, int *iters)

@@ -24,16 +24,26 @@
 //
 // What bounds it: HBM at N = 12 (64 B a node Poisson, 72 B Helmholtz), where
 // the 16-line tiles and the 4-steps fit the order exactly and every factor
-// load is four whole 128 B lines.  8000 elements: Poisson 238 -> 150 us (5.9
-// TB/s), Helmholtz 235 -> 166 us (6.0 TB/s), a Helmholtz CG iteration 475
-// -> 417 us.  It needs six (OP 0: seven) wavefronts a SIMD there: with five,
-// the two workgroups of nine do not spread over the four SIMDs, 195 us.
+// load is four whole 128 B lines.  8000 elements, launched back to back:
+// Poisson 238 -> 145-150 us (5.9-6.1 TB/s), Helmholtz 235 -> 166 us (6.0
+// TB/s); in the assembled operator, with the DSS after it, the Helmholtz one
+// takes 190 us (5.2 TB/s).  A Helmholtz CG iteration 475 -> 417 us.  It needs six (OP 0: seven) wavefronts a SIMD there: with
+// five, the two workgroups of nine do not spread over the four SIMDs, 195 us.
 // At N = 9 to 11 a fifth to a third of each tile and of the lanes is padding
 // and the factor rows straddle lines: on large meshes the team kernel is the
 // faster one (N = 10, 9216 elements: 135 us, here 133-155).  On small ones
-// the short chain of phases counts: N = 10 64 elements 10.8 -> 7 us, 512
-// elements 14.0 -> 9.0 us, a CG iteration there 34 -> 28 us; 1000 elements
-// 17.1 / 16.5-17.8 us (N = 9: 12.1 / 17.0), so the line is drawn at 512.
+// the short chain of phases counts, up to 512 elements at each of the three
+// orders; us, team / here (Poisson, Helmholtz, a Helmholtz CG iteration):
+//   elements       64                    512                   729
+//   N =  9   7.5/6.0 7.4/6.1    9.3/8.5  9.3/8.8    10.0/10.4 10.0/14.0
+//            18.6/15.6          25.7/24.7           28.1/30.9
+//   N = 10  10.8/6.0 8.9/6.1   13.7/9.1 13.1/9.6    14.8/13.3 14.3/13.9
+//            20.2/15.5          30.8/26.6           35.4/34.5
+//   N = 11  10.3/6.3 10.7/6.4  13.8/10.8 13.6/11.8  16.1/16.4 16.5/16.8
+//            22.3/16.6          34.7/30.4           41.7/38.9
+// At 1000 elements it loses at N = 9 (11.9 / 18.0 Helmholtz) and 11 (19.1 /
+// 21.2).  N = 13 needs 11 wavefronts and spills: 198 -> 239-278 us on a large
+// mesh; 14 to 16 were not tried.
 // Other lane layouts tried at N = 10 and 12: nodes in storage order in the
 // flux phase with the zeta product through LDS too (N = 12 213 us).
 #ifndef SSX_AXM_H
